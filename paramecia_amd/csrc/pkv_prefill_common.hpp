@@ -4,9 +4,9 @@
 // chosen to fill about 256 workgroups) and the kernel that merges the key splits' (m, l,
 // o) partials. Include-only; every symbol has internal linkage.
 //
-// Partial layout: part[batch * nsplit + split][kv head][pos * 8 + head of the group][258]:
-// entries 0-255 in tile order (entry i holds element tile_e(i / 16, i % 16)), then the
-// row's running max m (log2 units) and sum l.
+// Partial layout: part[batch * nsplit + split][kv head][pos * 8 + head of the group][256] in
+// tile order (entry i holds element tile_e(i / 16, i % 16)), and ml[same rows]: the row's
+// running max m (log2 units) and sum l.
 #pragma once
 #include "pkv_decode_split.hpp"
 
@@ -19,7 +19,8 @@ constexpr int kPosPerWG = 16;  // query positions per workgroup, two per wave
 constexpr int kRaw = 3;        // raw block stages in flight
 constexpr int kPfTargetWGs = 256;
 constexpr float kPfLazy = 8.0f;
-constexpr int kMaxMergeSplits = 16;
+constexpr int kNarrowSplits = 16;    // splits the narrow merge takes (all loads in flight)
+constexpr int kMaxMergeSplits = 128;  // splits the wide merge takes
 
 struct PrefillArgs {
   const float *q;  // [B][l][16][256]
@@ -28,10 +29,14 @@ struct PrefillArgs {
   int64_t seq_k;     // keys in the cache
   int64_t q_offset;  // query i sees key j iff !causal || j <= i + q_offset
   int l, causal;
-  int ntiles, nsplit, bps;  // position tiles, key splits, blocks per split
+  int ntiles, nsplit;  // position tiles; key splits of a tile, each its even share of the
+                       // blocks the tile sees (shares of the whole range left the last
+                       // splits of a prompt's first tiles empty: 2048 tokens 180 us at 2
+                       // splits, 118 us with even ones)
   int ngroups;              // (batch, split, KV head) groups: 2 * nsplit * batch
   float sl2;                // scale * log2(e)
-  float *part;  // [B * nsplit][2][l * 8][258] partials in tile order (nsplit > 1)
+  float *part;  // [B * nsplit][2][l * 8][256] partials in tile order (nsplit > 1)
+  float2 *ml;   // [B * nsplit][2][l * 8] their (m, l)
   float *out;   // [B][l][16][256] (nsplit == 1)
 };
 
@@ -40,50 +45,54 @@ struct PrefillArgs {
 // groups. The dispatcher deals workgroups to the 8 XCDs round-robin, so with 8 groups
 // (the 512-token chunk: 2 KV heads x 4 splits) every workgroup that streams one group's
 // key range runs on one XCD and the range is fetched into that XCD's L2 once, not by all
-// eight.
+// eight. The tiles go out last first: under the causal limit the last tile sees the most
+// keys, and the workgroups dispatched last then are the short ones (a 4001-token prompt,
+// 502 workgroups of 1 to 126 blocks on 256 CUs: 451 -> 316 us).
 struct PfWork {
   int tile, kvg, split, b;
 };
 __device__ __forceinline__ PfWork prefill_work(const PrefillArgs &a) {
   const int L = blockIdx.x, grp = L % a.ngroups, z = grp >> 1;
-  return PfWork{L / a.ngroups, grp & 1, z % a.nsplit, z / a.nsplit};
+  return PfWork{a.ntiles - 1 - L / a.ngroups, grp & 1, z % a.nsplit, z / a.nsplit};
 }
 
 // Merge the key splits: out[b][pos][8 kvg + hh][e] = sum_s o_s 2^(m_s - M) / sum_s l_s 2^(m_s - M).
 // One workgroup of 256 threads per 8 rows and batch: 32 threads per row, each taking 8
 // consecutive tile-order entries; every split's (m, l) and entries are loaded before any
-// is used (nsplit <= kMaxMergeSplits).
-__global__ __launch_bounds__(256) void prefill_merge_kernel(const float *part, int nsplit,
-                                                                int l, float *out) {
+// is used (nsplit <= kNarrowSplits).
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const float *part, const float2 *pml,
+                                                            int nsplit, int l, float *out) {
   const int r8 = threadIdx.x >> 5, j = threadIdx.x & 31;
   const int row = blockIdx.x * 8 + r8, b = blockIdx.y;  // row = kvg * l * 8 + pos * 8 + hh
   if (row >= 2 * l * 8) return;
   const int kvg = row / (l * 8), rr = row % (l * 8), pos = rr >> 3, hh = rr & 7;
-  const int64_t split_stride = (int64_t)2 * l * 8 * 258;
-  const float *base = part + (((int64_t)(b * nsplit) * 2 + kvg) * l * 8 + rr) * 258;
-  float2 ml[kMaxMergeSplits], v[kMaxMergeSplits][4];
+  const int64_t split_rows = (int64_t)2 * l * 8, row0 = (int64_t)b * nsplit * split_rows + row;
+  float2 ml[kNarrowSplits];
+  float4 v[kNarrowSplits][2];
 #pragma unroll
-  for (int s = 0; s < kMaxMergeSplits; ++s) {
+  for (int s = 0; s < kNarrowSplits; ++s) {
     if (s < nsplit) {
-      const float *pr = base + s * split_stride;
-      ml[s] = *reinterpret_cast<const float2 *>(pr + 256);
+      const int64_t r = row0 + s * split_rows;
+      ml[s] = pml[r];
 #pragma unroll
-      for (int k = 0; k < 4; ++k) v[s][k] = *reinterpret_cast<const float2 *>(pr + 8 * j + 2 * k);
+      for (int k = 0; k < 2; ++k) v[s][k] = *reinterpret_cast<const float4 *>(part + r * 256 + 8 * j + 4 * k);
     }
   }
   float M = -INFINITY;
 #pragma unroll
-  for (int s = 0; s < kMaxMergeSplits; ++s)
+  for (int s = 0; s < kNarrowSplits; ++s)
     if (s < nsplit) M = fmaxf(M, ml[s].x);
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, L = 0.0f;
 #pragma unroll
-  for (int s = 0; s < kMaxMergeSplits; ++s) {
+  for (int s = 0; s < kNarrowSplits; ++s) {
     if (s < nsplit) {
       const float f = (ml[s].x == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(ml[s].x - M);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        acc[2 * k] += f * v[s][k].x;
-        acc[2 * k + 1] += f * v[s][k].y;
+      for (int k = 0; k < 2; ++k) {
+        acc[4 * k] += f * v[s][k].x;
+        acc[4 * k + 1] += f * v[s][k].y;
+        acc[4 * k + 2] += f * v[s][k].z;
+        acc[4 * k + 3] += f * v[s][k].w;
       }
       L += f * ml[s].y;
     }
@@ -96,10 +105,112 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float *part, i
   }
 }
 
+// The same for up to kMaxMergeSplits splits (a short chunk over many keys): one workgroup
+// of 8 groups of 32 threads per row and batch. Group sg takes splits sg, sg + 8, ...: up
+// to 16 of them, every load issued before any is used; the groups' sums meet in LDS.
+__global__ __launch_bounds__(256) void prefill_merge_wide_kernel(const float *part,
+                                                                 const float2 *pml, int nsplit,
+                                                                 int l, float *out) {
+  constexpr int kPer = kMaxMergeSplits / 8;
+  __shared__ __attribute__((aligned(16))) float acc_s[8][256];
+  __shared__ float2 ml_s[8];
+  const int sg = threadIdx.x >> 5, j = threadIdx.x & 31;
+  const int row = blockIdx.x, b = blockIdx.y;
+  const int kvg = row / (l * 8), rr = row % (l * 8), pos = rr >> 3, hh = rr & 7;
+  const int64_t split_rows = (int64_t)2 * l * 8, row0 = (int64_t)b * nsplit * split_rows + row;
+  float2 ml[kPer];
+  float4 v[kPer][2];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    const int s = sg + 8 * i;
+    const bool ok = s < nsplit;  // past the splits: split 0's row, with no weight
+    const int64_t r = row0 + (ok ? s : 0) * split_rows;
+    const float2 t = pml[r];
+    ml[i] = ok ? t : float2{-INFINITY, 0.0f};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) v[i][k] = *reinterpret_cast<const float4 *>(part + r * 256 + 8 * j + 4 * k);
+  }
+  float m = -INFINITY;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) m = fmaxf(m, ml[i].x);
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, L = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    if (ml[i].x == -INFINITY) continue;
+    const float f = __builtin_amdgcn_exp2f(ml[i].x - m);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      acc[4 * k] += f * v[i][k].x;
+      acc[4 * k + 1] += f * v[i][k].y;
+      acc[4 * k + 2] += f * v[i][k].z;
+      acc[4 * k + 3] += f * v[i][k].w;
+    }
+    L += f * ml[i].y;
+  }
+  *reinterpret_cast<float4 *>(&acc_s[sg][8 * j]) = float4{acc[0], acc[1], acc[2], acc[3]};
+  *reinterpret_cast<float4 *>(&acc_s[sg][8 * j + 4]) = float4{acc[4], acc[5], acc[6], acc[7]};
+  if (j == 0) ml_s[sg] = float2{m, L};
+  __syncthreads();
+  float M = -INFINITY, Lt = 0.0f, o = 0.0f;
+#pragma unroll
+  for (int g = 0; g < 8; ++g) M = fmaxf(M, ml_s[g].x);
+  const int idx = threadIdx.x;
+#pragma unroll
+  for (int g = 0; g < 8; ++g) {
+    const float f = (ml_s[g].x == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(ml_s[g].x - M);
+    o += f * acc_s[g][idx];
+    Lt += f * ml_s[g].y;
+  }
+  out[(((int64_t)b * l + pos) * 16 + 8 * kvg + hh) * 256 + tile_e(idx >> 4, idx & 15)] =
+      Lt > 0.0f ? o / Lt : 0.0f;
+}
+
 }  // namespace
 
-// The plan of a prefill chunk over 32-key blocks: position tiles, key splits (enough
-// workgroups to fill the GPU, at most kMaxMergeSplits), the partials' workspace.
+// Bytes of an nsplit-way plan's partials.
+static inline size_t prefill_part_bytes(int batch, int nsplit, int l) {
+  return (size_t)batch * nsplit * 2 * l * 8 * 258 * sizeof(float);
+}
+
+// The number of key splits: the one with the least estimated time, in units of a block
+// (32 keys) of one workgroup, of which 256 run at a time (one per CU).
+//   rounds x (a workgroup's mean blocks + kPfFixed), or the longest workgroup's time where
+//   that is more, + the merge's time (its partials written and read once).
+// A chunk that fills the GPU by itself keeps one split; 512 tokens over 16896 keys take 4
+// (256 workgroups); a few tokens over a long cache take as many as give every CU a
+// workgroup: 5 tokens over 20016 keys ran 32 workgroups at the earlier limit of 16
+// splits, 98.8 us with the merge; at 128 splits 24.5 us.
+static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk, size_t limit) {
+  constexpr double kPfFixed = 2.0;   // q, the first block's latency, the epilogue
+  constexpr double kMergeFixed = 1.5, kMergeBytes = 7e6;  // bytes merged in a block's time
+  const int base = ntiles * 2 * a.batch;
+  // blocks of the first and the last tile (the causal limit cuts the first ones')
+  double b0 = nblk, b1 = nblk;
+  if (a.causal) {
+    auto seen = [&](int64_t keys) { return (double)((keys < a.seq_k ? keys : a.seq_k) + 31) / 32; };
+    b0 = seen(a.q_offset + (a.l < kPosPerWG ? a.l : kPosPerWG));
+    b1 = seen(a.q_offset + a.l);
+  }
+  const double mean = 0.5 * (b0 + b1);
+  int best = 1;
+  double best_t = 1e30;
+  for (int ns = 1; ns <= kMaxMergeSplits && ns <= (nblk > 0 ? nblk : 1); ++ns) {
+    const size_t bytes = ns > 1 ? prefill_part_bytes(a.batch, ns, a.l) : 0;
+    if (bytes > limit) break;
+    const int64_t rounds = ((int64_t)base * ns + kPfTargetWGs - 1) / kPfTargetWGs;
+    const double even = rounds * (mean / ns + kPfFixed), longest = b1 / ns + kPfFixed;
+    const double t = (even > longest ? even : longest) +
+                     (ns > 1 ? kMergeFixed + 2.0 * bytes / kMergeBytes : 0.0);
+    if (t < best_t) {
+      best_t = t;
+      best = ns;
+    }
+  }
+  return best;
+}
+
+// The plan of a prefill chunk over 32-key blocks: position tiles, key splits, the
+// partials' workspace.
 static inline int prefill_plan(const AttnArgs &a, float sl2, Workspace &ws, PrefillArgs &d) {
   d.q = a.q;
   d.k = a.k;
@@ -114,22 +225,31 @@ static inline int prefill_plan(const AttnArgs &a, float sl2, Workspace &ws, Pref
   d.sl2 = sl2;
   d.ntiles = (a.l + kPosPerWG - 1) / kPosPerWG;
   const int nblk = (int)((a.seq_k + 31) / 32);
-  const int base = d.ntiles * 2 * a.batch;
-  int nsplit = (kPfTargetWGs + base - 1) / base;
-  if (nsplit > kMaxMergeSplits) nsplit = kMaxMergeSplits;
-  if (nsplit > nblk) nsplit = nblk > 0 ? nblk : 1;
-  if (nsplit < 1) nsplit = 1;
-  d.bps = (nblk + nsplit - 1) / nsplit;
-  if (d.bps < 1) d.bps = 1;
+  size_t limit = ~(size_t)0;
+  if (ws.fixed) {
+    // A no-alloc call is accepted when 256 workgroups' worth of splits (16 at most) fit
+    // the scratch, and then takes no more splits than fit.
+    const int base = d.ntiles * 2 * a.batch;
+    int need = (kPfTargetWGs + base - 1) / base;
+    need = need > 16 ? 16 : need;
+    need = need > nblk ? (nblk > 0 ? nblk : 1) : need;
+    if (need > 1) {
+      const int rc = ws.reserve(prefill_part_bytes(a.batch, need, a.l));
+      if (rc) return rc;
+    }
+    limit = ws.bytes;
+  }
+  const int nsplit = prefill_splits(a, d.ntiles, nblk, limit);
   d.nsplit = nsplit;
   d.ngroups = 2 * nsplit * a.batch;
   d.out = a.out;
   d.part = nullptr;
+  d.ml = nullptr;
   if (nsplit > 1) {
-    const size_t need = (size_t)a.batch * nsplit * 2 * a.l * 8 * 258 * sizeof(float);
-    const int rc = ws.reserve(need);
+    const int rc = ws.reserve(prefill_part_bytes(a.batch, nsplit, a.l));
     if (rc) return rc;
     d.part = static_cast<float *>(ws.ptr);
+    d.ml = reinterpret_cast<float2 *>(d.part + (size_t)a.batch * nsplit * 2 * a.l * 8 * 256);
   }
   return PKV_OK;
 }
@@ -137,8 +257,12 @@ static inline int prefill_plan(const AttnArgs &a, float sl2, Workspace &ws, Pref
 // The split merge after a prefill kernel that wrote partials (nsplit > 1).
 static inline int prefill_merge(const PrefillArgs &d, int batch, hipStream_t s) {
   if (d.nsplit <= 1) return PKV_OK;
-  hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((2 * d.l * 8 + 7) / 8), (unsigned)batch),
-                     dim3(256), 0, s, d.part, d.nsplit, d.l, d.out);
+  if (d.nsplit <= kNarrowSplits)
+    hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((2 * d.l * 8 + 7) / 8), (unsigned)batch),
+                       dim3(256), 0, s, d.part, d.ml, d.nsplit, d.l, d.out);
+  else
+    hipLaunchKernelGGL(prefill_merge_wide_kernel, dim3((unsigned)(2 * d.l * 8), (unsigned)batch),
+                       dim3(256), 0, s, d.part, d.ml, d.nsplit, d.l, d.out);
   PKV_HIP(hipGetLastError());
   return PKV_OK;
 }

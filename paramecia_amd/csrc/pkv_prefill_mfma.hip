@@ -228,10 +228,14 @@ __global__ __launch_bounds__(kPfThreads) void q4k_prefill_kernel(PrefillArgs a) 
   const PfWork wk = prefill_work(a);
   const int tile = wk.tile, kvg = wk.kvg, split = wk.split, b = wk.b;
   const int p0 = tile * kPosPerWG;
-  const int pw = p0 + 2 * wave;  // this wave's first position; row n -> pw + n / 8
+  // this wave's first position (row n -> pw + n / 8). The last waves, which have the least
+  // to do besides the MFMAs, take the first positions; a wave without a position (the
+  // chunk's last tile) only builds operands.
+  const int pw = __builtin_amdgcn_readfirstlane(p0 + 2 * (kPfWaves - 1 - wave));
+  const bool active = pw < a.l;
 
-  // ---- key blocks of this workgroup: its split, cut at the last key any of its queries
-  // may see
+  // ---- key blocks of this workgroup: its split of the blocks up to the last key any of
+  // its tile's queries may see
   int64_t kend = a.seq_k;
   if (a.causal) {
     const int64_t plast = (p0 + kPosPerWG - 1 < a.l ? p0 + kPosPerWG - 1 : a.l - 1);
@@ -239,8 +243,9 @@ __global__ __launch_bounds__(kPfThreads) void q4k_prefill_kernel(PrefillArgs a) 
     if (lim < kend) kend = lim;
   }
   const int nblk_all = (int)((kend + kBlk - 1) / kBlk);
-  const int kb0 = split * a.bps;
-  const int kb1 = kb0 + a.bps < nblk_all ? kb0 + a.bps : nblk_all;
+  const int bps = (nblk_all + a.nsplit - 1) / a.nsplit;
+  const int kb0 = split * bps;
+  const int kb1 = kb0 + bps < nblk_all ? kb0 + bps : nblk_all;
   const int nb = kb1 > kb0 ? kb1 - kb0 : 0;
 
   const uint8_t *kbase = a.k + b * a.rs_b + kvg * a.rs_h;
@@ -335,7 +340,7 @@ __global__ __launch_bounds__(kPfThreads) void q4k_prefill_kernel(PrefillArgs a) 
     dequant(0);
     if (wave == 4) dequant_mins(0);
   }
-  for (int i = 0; i < nb; ++i) {
+  auto next_block = [&](int i) {
     if (loader && i + 1 < nb) {  // block i + 1 landed (block i + 2 may still fly)
       if (i + 2 < nb)  // the 6 loads of block i + 2 may stay in flight
         asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
@@ -347,6 +352,16 @@ __global__ __launch_bounds__(kPfThreads) void q4k_prefill_kernel(PrefillArgs a) 
     __syncthreads();
     if (loader && i + 3 < nb) issue(i + 3);
     if (i + 1 < nb) dequant(i + 1);
+  };
+  if (!active) {
+    for (int i = 0; i < nb; ++i) {
+      next_block(i);
+      if (wave == 4 && i + 1 < nb) dequant_mins(i + 1);
+    }
+    return;
+  }
+  for (int i = 0; i < nb; ++i) {
+    next_block(i);
     const DqBlock &D = sm.dq[i & 1];
 
     // ---- QK (two tiles of 16 keys), rows = this wave's 16 query rows; keys kk of the
@@ -481,22 +496,20 @@ __global__ __launch_bounds__(kPfThreads) void q4k_prefill_kernel(PrefillArgs a) 
       }
     }
   } else {
-    float *pz = a.part + (((int64_t)(b * a.nsplit + split) * 2 + kvg) * a.l * 8) * 258;
+    const int64_t r0 = ((int64_t)(b * a.nsplit + split) * 2 + kvg) * a.l * 8;
 #pragma unroll
     for (int ii = 0; ii < 4; ++ii) {
       const int row = 4 * g + ii;
       const int pos = pw + (row >> 3);
       if (pos >= a.l) continue;
-      float *prow = pz + ((int64_t)pos * 8 + (row & 7)) * 258;
+      const int64_t r = r0 + (int64_t)pos * 8 + (row & 7);
+      float *prow = a.part + r * 256;
 #pragma unroll
       for (int T2 = 0; T2 < 16; ++T2) {
         const int e = tile_e(T2, n);
         prow[16 * T2 + n] = acc[T2][ii] - cmin[row][e >> 5];
       }
-      if (n == 0) {
-        prow[256] = mrow[ii];
-        prow[257] = lrow[ii];
-      }
+      if (n == 0) a.ml[r] = float2{mrow[ii], lrow[ii]};
     }
   }
 }

@@ -160,10 +160,14 @@ __global__ __launch_bounds__(kPfThreads) void q8_prefill_kernel(PrefillArgs a) {
   const PfWork wk = prefill_work(a);
   const int tile = wk.tile, kvg = wk.kvg, split = wk.split, b = wk.b;
   const int p0 = tile * kPosPerWG;
-  const int pw = p0 + 2 * wave;  // this wave's first position; row n -> pw + n / 8
+  // this wave's first position (row n -> pw + n / 8). The last waves, which have the least
+  // to do besides the MFMAs, take the first positions; a wave without a position (the
+  // chunk's last tile) only builds operands.
+  const int pw = __builtin_amdgcn_readfirstlane(p0 + 2 * (kPfWaves - 1 - wave));
+  const bool active = pw < a.l;
 
-  // ---- key blocks of this workgroup: its split, cut at the last key any of its queries
-  // may see
+  // ---- key blocks of this workgroup: its split of the blocks up to the last key any of
+  // its tile's queries may see
   int64_t kend = a.seq_k;
   if (a.causal) {
     const int64_t plast = (p0 + kPosPerWG - 1 < a.l ? p0 + kPosPerWG - 1 : a.l - 1);
@@ -171,8 +175,9 @@ __global__ __launch_bounds__(kPfThreads) void q8_prefill_kernel(PrefillArgs a) {
     if (lim < kend) kend = lim;
   }
   const int nblk_all = (int)((kend + kBlk - 1) / kBlk);
-  const int kb0 = split * a.bps;
-  const int kb1 = kb0 + a.bps < nblk_all ? kb0 + a.bps : nblk_all;
+  const int bps = (nblk_all + a.nsplit - 1) / a.nsplit;
+  const int kb0 = split * bps;
+  const int kb1 = kb0 + bps < nblk_all ? kb0 + bps : nblk_all;
   const int nb = kb1 > kb0 ? kb1 - kb0 : 0;
 
   const uint8_t *kbase = a.k + b * a.rs_b + kvg * a.rs_h;
@@ -267,6 +272,10 @@ __global__ __launch_bounds__(kPfThreads) void q8_prefill_kernel(PrefillArgs a) {
     __syncthreads();
     if (loader && i + 3 < nb) issue(i + 3);
     if (i + 1 < nb && !late) dequant(i + 1);
+    if (!active) {
+      if (i + 1 < nb && late) dequant(i + 1);
+      continue;
+    }
     const Q8Dq &D = sm.dq[i & 1];
 
     // ---- QK (two tiles of 16 keys); keys of the block at or past nlim are masked (past
@@ -342,6 +351,8 @@ __global__ __launch_bounds__(kPfThreads) void q8_prefill_kernel(PrefillArgs a) {
     if (i + 1 < nb && late) dequant(i + 1);
   }
 
+  if (!active) return;
+
   // ---- epilogue: row sums, then the output or the split's partial
   lsum += __shfl_xor(lsum, 16);
   lsum += __shfl_xor(lsum, 32);
@@ -363,19 +374,17 @@ __global__ __launch_bounds__(kPfThreads) void q8_prefill_kernel(PrefillArgs a) {
       for (int T = 0; T < 16; ++T) orow[tile_e(T, n)] = acc[T][ii] * inv;
     }
   } else {
-    float *pz = a.part + (((int64_t)(b * a.nsplit + split) * 2 + kvg) * a.l * 8) * 258;
+    const int64_t r0 = ((int64_t)(b * a.nsplit + split) * 2 + kvg) * a.l * 8;
 #pragma unroll
     for (int ii = 0; ii < 4; ++ii) {
       const int row = 4 * g + ii;
       const int pos = pw + (row >> 3);
       if (pos >= a.l) continue;
-      float *prow = pz + ((int64_t)pos * 8 + (row & 7)) * 258;
+      const int64_t r = r0 + (int64_t)pos * 8 + (row & 7);
+      float *prow = a.part + r * 256;
 #pragma unroll
       for (int T = 0; T < 16; ++T) prow[16 * T + n] = acc[T][ii];
-      if (n == 0) {
-        prow[256] = mrow[ii];
-        prow[257] = lrow[ii];
-      }
+      if (n == 0) a.ml[r] = float2{mrow[ii], lrow[ii]};
     }
   }
 }

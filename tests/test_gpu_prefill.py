@@ -98,6 +98,17 @@ def test_prefill_unsplit(pk, orc, quant):
 
 
 @pytest.mark.parametrize("quant", QUANTS)
+@pytest.mark.parametrize("S,L,causal", [(20000, 5, True), (3001, 2, True), (600, 18, True),
+                                        (530, 16, False), (0, 1000, True), (0, 2048, False)])
+def test_prefill_split_plan(pk, orc, S, L, causal, quant):
+    """The key split's range: 128 splits and fewer through the wide merge (17 or more), a
+    last tile with one wave's positions, the narrow merge (3 splits of unequal tiles), and
+    a chunk that fills the GPU unsplit."""
+    say(f"prefill split plan quant={quant} S={S} L={L} causal={causal}")
+    run_prefill(pk, orc, S, L, causal=causal, seed=S + L, quant=quant)
+
+
+@pytest.mark.parametrize("quant", QUANTS)
 def test_prefill_outlier_channels(pk, orc, quant):
     say(f"prefill outlier channels quant={quant}")
     from paramecia_amd import workloads as W
