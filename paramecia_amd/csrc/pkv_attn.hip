@@ -28,6 +28,13 @@ int launch_append_attend_batched_q8(int quant, const SeqDesc *seqs, int n, const
                                     const float *v, const float *q, int num_heads,
                                     int num_kv_heads, int head_dim, float scale, float *out,
                                     Workspace &ws, hipStream_t s);
+// F16 / BF16 decode for the Qwen3-Next shape (pkv_half_decode.hip).
+int launch_attend_half(const AttnArgs &a, const float *k_new, const float *v_new, uint8_t *kc,
+                       uint8_t *vc, int64_t t_new, Workspace &ws, hipStream_t s);
+int launch_append_attend_batched_half(int quant, const SeqDesc *seqs, int n, const float *k,
+                                      const float *v, const float *q, int num_heads,
+                                      int num_kv_heads, int head_dim, float scale, float *out,
+                                      Workspace &ws, hipStream_t s);
 // Prefill chunk (l > 1) over Q4K rows of the Qwen3-Next shape (pkv_prefill_mfma.hip).
 int launch_prefill_mfma(const AttnArgs &a, Workspace &ws, hipStream_t s);
 int launch_prefill_q8_mfma(const AttnArgs &a, Workspace &ws, hipStream_t s);
@@ -175,21 +182,31 @@ int launch_generic_g(const AttnArgs &a, int R, dim3 grid, int64_t kpw, int wpg, 
 
 }  // namespace
 
-int launch_attend_generic(const AttnArgs &a, Workspace &ws, hipStream_t s) {
-  const int G = a.num_heads / a.num_kv_heads;
-  const int R = a.head_dim <= 64 ? 1 : a.head_dim <= 128 ? 2 : a.head_dim <= 256 ? 4 : 8;
+// Waves per (batch row, query, KV head): enough to fill the GPU, at least 16 keys each.
+static int64_t generic_waves(const AttnArgs &a) {
   const int groups = a.batch * a.l * a.num_kv_heads;
-  // Enough waves to fill the GPU, at least 16 keys per wave.
   int64_t want = (16384 + groups - 1) / groups;
   if (want > 4096) want = 4096;  // combine keeps one weight per split in LDS
   int64_t max_waves = (a.seq_k + 15) / 16;
   int64_t wpg = want < max_waves ? want : max_waves;
   wpg = (wpg + kWaves - 1) / kWaves * kWaves;
-  if (wpg < kWaves) wpg = kWaves;
+  return wpg < kWaves ? kWaves : wpg;
+}
+static size_t generic_bytes(const AttnArgs &a) {
+  const int rows = a.batch * a.l * a.num_heads;
+  return (size_t)generic_waves(a) * rows * (2 + (size_t)a.head_dim) * sizeof(float);
+}
+
+int generic_plan_fits(const AttnArgs &a, Workspace &ws) { return ws.reserve(generic_bytes(a)); }
+
+int launch_attend_generic(const AttnArgs &a, Workspace &ws, hipStream_t s) {
+  const int G = a.num_heads / a.num_kv_heads;
+  const int R = a.head_dim <= 64 ? 1 : a.head_dim <= 128 ? 2 : a.head_dim <= 256 ? 4 : 8;
+  const int groups = a.batch * a.l * a.num_kv_heads;
+  const int64_t wpg = generic_waves(a);
   const int64_t kpw = (a.seq_k + wpg - 1) / wpg;
   const int rows = a.batch * a.l * a.num_heads;
-  const size_t need = (size_t)wpg * rows * (2 + (size_t)a.head_dim) * sizeof(float);
-  int rc = ws.reserve(need);
+  int rc = ws.reserve(generic_bytes(a));
   if (rc) return rc;
   Partials P;
   P.m = reinterpret_cast<float *>(ws.ptr);
@@ -230,6 +247,8 @@ int launch_attend(const AttnArgs &a, Workspace &ws, hipStream_t s) {
   if (rc != PKV_ERR_UNSUPPORTED) return rc;
   rc = launch_attend_q8(a, nullptr, nullptr, nullptr, nullptr, -1, ws, s);
   if (rc != PKV_ERR_UNSUPPORTED) return rc;
+  rc = launch_attend_half(a, nullptr, nullptr, nullptr, nullptr, -1, ws, s);
+  if (rc != PKV_ERR_UNSUPPORTED) return rc;
   rc = launch_prefill_mfma(a, ws, s);
   if (rc != PKV_ERR_UNSUPPORTED) return rc;
   rc = launch_prefill_q8_mfma(a, ws, s);
@@ -245,6 +264,8 @@ int launch_append_attend(const AttnArgs &a, const float *k_new, const float *v_n
   rc = launch_attend_mfma(a, k_new, v_new, kc, vc, t_new, ws, s);
   if (rc != PKV_ERR_UNSUPPORTED) return rc;
   rc = launch_attend_q8(a, k_new, v_new, kc, vc, t_new, ws, s);
+  if (rc != PKV_ERR_UNSUPPORTED) return rc;
+  rc = launch_attend_half(a, k_new, v_new, kc, vc, t_new, ws, s);
   if (rc != PKV_ERR_UNSUPPORTED) return rc;
   rc = launch_append(a.quant, k_new, v_new, kc, vc, a.batch, a.num_kv_heads, a.head_dim, 1,
                      t_new, s);
@@ -263,6 +284,9 @@ int launch_append_attend_batched(int quant, const SeqDesc *seqs, int n, const fl
   const int rc1 = launch_append_attend_batched_q8(quant, seqs, n, k, v, q, num_heads,
                                                   num_kv_heads, head_dim, scale, out, ws, s);
   if (rc1 != PKV_ERR_UNSUPPORTED) return rc1;
+  const int rc2 = launch_append_attend_batched_half(quant, seqs, n, k, v, q, num_heads,
+                                                    num_kv_heads, head_dim, scale, out, ws, s);
+  if (rc2 != PKV_ERR_UNSUPPORTED) return rc2;
   const size_t kv_stride = (size_t)num_kv_heads * head_dim;
   const size_t q_stride = (size_t)num_heads * head_dim;
   const int64_t bpr = (int64_t)row_bytes(quant, head_dim);
