@@ -19,6 +19,7 @@
 
 #include "pkv_internal.hpp"
 #include "pkv_scalar.hpp"
+#include "pkv_q4k_fit.hpp"
 #include "pkv_q4k_lanes.hpp"
 #include "pkv_prep_common.hpp"
 
@@ -184,6 +185,224 @@ __global__ __launch_bounds__(kPrepThreads) void prep_append_kernel(PrepArgs a, i
   }
 }
 
+// ---- many rows (head_dim 256): tiles of rows per workgroup
+//
+// The row kernel above has one lane add a row's 256 squares in order while the other 63
+// (a K row: 255) wait, and quantizes a K or V row as one latency chain: 145 us for 4001
+// tokens, of which the bytes (147 MB) take about 30 at the copy rate. Here a workgroup takes a tile of rows
+// of one kind; the squares of the tile go to LDS and lane r adds those of row r, so the
+// ordered sums of all its rows run side by side; the normalised rows are quantized with 8
+// kL lanes per row, as pkv_append does (kL from the row count, by the same limits).
+// 4001 tokens: 136 -> 42 us Q4K, 66 -> 37 us Q8_0 and F16.
+// Rows (q, K and V) from which the tiles are used, and superblocks up to which a K or V
+// superblock takes 4 lanes per sub-block (2 above). Model shape, us, rows kernel / tiles:
+// Q4K 1 token 7.8 / 7.9, 5 tokens 8.0 / 7.6, 512 25.1 / 10.3; Q8_0 256 tokens 7.6 / 10.3,
+// 512 12.4 / 11.0; F16 512 11.7 / 10.9. 4 lanes against 2: 512 tokens 10.4 / 12.9, 1024
+// tokens 17.2 / 15.1.
+constexpr int64_t kTileMinRowsQ4K = 40, kTileMinRowsOther = 10240, kFit4Blocks = 2048;
+constexpr int kTileRows = 16;   // rows of a tile (K and V of few rows: 8)
+constexpr int kTileStride = 260;  // floats per LDS row: b128 reads of 8 rows on 32 banks
+
+// Normalise and rotate the kN rows a wave holds in x (lane l: elements 4 l .. 4 l + 3 of row
+// r0 + i), with the arithmetic of prep_row. Every wave of the workgroup calls it.
+template <int kN>
+__device__ __forceinline__ void prep_tile(float4 (&x)[kN], float (*rows)[kTileStride], float *m,
+                                          int r0, int nrows, int tid, float4 alpha, float eps,
+                                          int n_rot, const float *cos_tab, const float *sin_tab,
+                                          const int64_t (&pos)[kN]) {
+#pragma clang fp contract(off)
+  const int lane = tid & 63, half = n_rot >> 1;
+  // the rotation's cos and sin, loaded ahead of the sums: elements 4 lane .. + 3
+  const bool rot = 4 * lane < n_rot;
+  float cs[kN][4], sn[kN][4];
+#pragma unroll
+  for (int i = 0; i < kN; ++i)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int e = 4 * lane + k, j = e < half ? e : e - half;
+      const bool in = rot && e < n_rot;
+      cs[i][k] = in ? cos_tab[pos[i] * half + j] : 1.0f;
+      sn[i][k] = in ? sin_tab[pos[i] * half + j] : 0.0f;
+    }
+#pragma unroll
+  for (int i = 0; i < kN; ++i)
+    *reinterpret_cast<float4 *>(&rows[r0 + i][4 * lane]) =
+        float4{x[i].x * x[i].x, x[i].y * x[i].y, x[i].z * x[i].z, x[i].w * x[i].w};
+  __syncthreads();
+  if (tid < nrows) {
+    float sum2 = -0.0f;
+#pragma unroll 16
+    for (int e = 0; e < 64; ++e) {
+      const float4 t = *reinterpret_cast<const float4 *>(&rows[tid][4 * e]);
+      sum2 += t.x;
+      sum2 += t.y;
+      sum2 += t.z;
+      sum2 += t.w;
+    }
+    m[tid] = __builtin_sqrtf(sum2 / 256.0f + eps);
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kN; ++i) {
+    const float mm = m[r0 + i];
+    x[i].x = x[i].x / mm * alpha.x;
+    x[i].y = x[i].y / mm * alpha.y;
+    x[i].z = x[i].z / mm * alpha.z;
+    x[i].w = x[i].w / mm * alpha.w;
+  }
+  if (n_rot == 0) return;
+  // the rotated elements through the wave's own LDS rows
+#pragma unroll
+  for (int i = 0; i < kN; ++i)
+    if (rot) *reinterpret_cast<float4 *>(&rows[r0 + i][4 * lane]) = x[i];
+  __builtin_amdgcn_wave_barrier();
+  if (rot) {
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const float *row = rows[r0 + i];
+      float v[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int e = 4 * lane + k;
+        if (e < half)
+          v[k] = v[k] * cs[i][k] - row[e + half] * sn[i][k];
+        else if (e < n_rot)
+          v[k] = row[e - half] * sn[i][k] + v[k] * cs[i][k];
+      }
+      x[i] = float4{v[0], v[1], v[2], v[3]};
+    }
+  }
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Positions of rows r .. r + kN - 1 of a [batch, l, heads] order: two divisions, then steps
+// (a 64-bit division per row took longer than the rest of a tile).
+template <int kN>
+__device__ __forceinline__ void tile_pos(uint32_t r, uint32_t heads, uint32_t l, int64_t t0,
+                                         int64_t (&pos)[kN]) {
+  uint32_t bt = r / heads, h = r - bt * heads, t = bt % l;
+#pragma unroll
+  for (int i = 0; i < kN; ++i) {
+    pos[i] = t0 + t;
+    if (++h == heads) {
+      h = 0;
+      t = t + 1 == l ? 0 : t + 1;
+    }
+  }
+}
+
+enum { kTileQ4K, kTileQ8, kTileHalf };
+
+// Workgroups [0, kv_wgs) take K tiles, [kv_wgs, 2 kv_wgs) V tiles (the quantizers are the
+// long ones), the rest q tiles.
+template <int kFmt, int kL>
+__global__ __launch_bounds__(256) void prep_tiles_kernel(PrepArgs a, uint32_t kv_wgs) {
+#pragma clang fp contract(off)
+  __shared__ __attribute__((aligned(16))) float rows[kTileRows][kTileStride];
+  __shared__ float m[kTileRows];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t wg = blockIdx.x;
+  if (wg >= 2 * kv_wgs) {
+    constexpr int kN = kTileRows / 4;
+    const int64_t base = (int64_t)(wg - 2 * kv_wgs) * kTileRows;
+    const int r0 = kN * wave;
+    float4 x[kN];
+    int64_t pos[kN];
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {  // rows past the last read it again and are not stored
+      int64_t r = base + r0 + i;
+      r = r < a.q_rows ? r : a.q_rows - 1;
+      x[i] = reinterpret_cast<const float4 *>(a.q + r * 256)[lane];
+    }
+    tile_pos<kN>((uint32_t)(base + r0), (uint32_t)a.num_heads, (uint32_t)a.l, a.t0, pos);
+    prep_tile<kN>(x, rows, m, r0, kTileRows, tid, reinterpret_cast<const float4 *>(a.q_alpha)[lane],
+                  a.eps, a.n_rot, a.cos_tab, a.sin_tab, pos);
+#pragma unroll
+    for (int i = 0; i < kN; ++i)
+      if (base + r0 + i < a.q_rows)
+        reinterpret_cast<float4 *>(a.q_out + (base + r0 + i) * 256)[lane] = x[i];
+    return;
+  }
+  constexpr int kR = kFmt == kTileQ4K && kL == 4 ? 8 : kTileRows, kN = kR / 4;  // of the tile, per wave
+  const bool is_v = wg >= kv_wgs;
+  const int64_t base = (int64_t)(is_v ? wg - kv_wgs : wg) * kR;
+  const float *src = is_v ? a.v : a.k;
+  const int r0 = kN * wave;
+  float4 x[kN];
+  int64_t pos[kN];
+#pragma unroll
+  for (int i = 0; i < kN; ++i) {
+    int64_t r = base + r0 + i;
+    r = r < a.kv_rows ? r : a.kv_rows - 1;
+    x[i] = reinterpret_cast<const float4 *>(src + r * 256)[lane];
+  }
+  tile_pos<kN>((uint32_t)(base + r0), (uint32_t)a.kv_heads, (uint32_t)a.l, a.t0, pos);
+  if (!is_v)
+    prep_tile<kN>(x, rows, m, r0, kR, tid, reinterpret_cast<const float4 *>(a.k_alpha)[lane], a.eps,
+                  a.n_rot, a.cos_tab, a.sin_tab, pos);
+  // destination row of source row r = (b * l + t) * kv_heads + h
+  auto dst_row = [&](int64_t row) {
+    const uint32_t r = (uint32_t)row, hs = (uint32_t)a.kv_heads, l = (uint32_t)a.l;
+    const uint32_t bt = r / hs, b = bt / l, t = bt - b * l;
+    return (is_v ? a.vc : a.kc) + (((a.t0 + t) * a.batch + b) * a.kv_heads + (r - bt * hs)) * a.bpr;
+  };
+  if constexpr (kFmt == kTileHalf) {
+    const bool bf = a.quant == PKV_QUANT_BF16;
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+      const float v[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
+      uint16_t y[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) y[k] = bf ? f32_to_bf16(v[k]) : f32_to_f16(v[k]);
+      if (base + r0 + i < a.kv_rows)
+        reinterpret_cast<uint2 *>(dst_row(base + r0 + i))[lane] =
+            uint2{(uint32_t)y[0] | ((uint32_t)y[1] << 16), (uint32_t)y[2] | ((uint32_t)y[3] << 16)};
+    }
+  } else {
+  // the quantizers: 8 kL lanes per row, each with 32 / kL elements in order
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < kN; ++i) *reinterpret_cast<float4 *>(&rows[r0 + i][4 * lane]) = x[i];
+  __syncthreads();
+  constexpr int E = 32 / kL;
+  // (Q8_0: the threads past the tile's blocks leave; no barrier follows)
+  const int rr = tid / (8 * kL), r = tid & (8 * kL - 1);
+  if (rr >= kR) return;
+  float y[E];
+#pragma unroll
+  for (int i = 0; i < E / 4; ++i) {
+    const float4 t = *reinterpret_cast<const float4 *>(&rows[rr][E * r + 4 * i]);
+    y[4 * i] = t.x;
+    y[4 * i + 1] = t.y;
+    y[4 * i + 2] = t.z;
+    y[4 * i + 3] = t.w;
+  }
+  const bool live = base + rr < a.kv_rows;
+  uint8_t *dst = dst_row(live ? base + rr : a.kv_rows - 1);
+  if constexpr (kFmt == kTileQ4K) {
+    q4k_quantize_group<kL>(y, r, dst, live);
+  } else {  // one lane per block
+    static_assert(kL == 1, "Q8_0: one lane per block");
+    float amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) amax = fmax_rs(amax, __builtin_fabsf(y[i]));
+    const float d = amax / 127.0f;
+    const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
+    uint16_t w[17];
+    w[0] = f32_to_f16(d);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      w[1 + i] = (uint16_t)((uint32_t)(uint8_t)rs_as_i8(__builtin_roundf(y[2 * i] * id)) |
+                            ((uint32_t)(uint8_t)rs_as_i8(__builtin_roundf(y[2 * i + 1] * id)) << 8));
+    if (live) {
+      uint16_t *o = reinterpret_cast<uint16_t *>(dst + 34 * r);
+#pragma unroll
+      for (int i = 0; i < 17; ++i) o[i] = w[i];
+    }
+  }
+  }
+}
+
 }  // namespace
 
 int launch_prep_append(const PrepArgs &a, hipStream_t s) {
@@ -193,6 +412,29 @@ int launch_prep_append(const PrepArgs &a, hipStream_t s) {
   const int64_t grid = q_wgs + 2 * a.kv_rows;
   if (grid == 0) return PKV_OK;
   if (grid >= (1ll << 31)) return set_error(PKV_ERR_ARG, "too many rows in one append");
+  // Tiles where the rows are many and the loads may be 16 bytes wide, four elements a lane.
+  const uintptr_t ptrs = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.q_out) |
+                         reinterpret_cast<uintptr_t>(a.k) | reinterpret_cast<uintptr_t>(a.v) |
+                         reinterpret_cast<uintptr_t>(a.q_alpha) |
+                         reinterpret_cast<uintptr_t>(a.k_alpha);
+  const bool q4 = a.quant == PKV_QUANT_Q4K;
+  if (a.head_dim == 256 && (ptrs & 15) == 0 && a.kv_rows > 0 && a.q_rows < (1ll << 31) &&
+      a.q_rows + 2 * a.kv_rows >= (q4 ? kTileMinRowsQ4K : kTileMinRowsOther)) {
+    const int kl = !q4 ? 1 : a.kv_rows * 2 <= kFit4Blocks ? 4 : 2;
+    const int64_t per = kl == 4 ? 8 : kTileRows, kv_wgs = (a.kv_rows + per - 1) / per;
+    const dim3 g((unsigned)(2 * kv_wgs + (a.q_rows + kTileRows - 1) / kTileRows)), t(256);
+    const uint32_t kw = (uint32_t)kv_wgs;
+    if (q4 && kl == 4)
+      hipLaunchKernelGGL((prep_tiles_kernel<kTileQ4K, 4>), g, t, 0, s, a, kw);
+    else if (q4)
+      hipLaunchKernelGGL((prep_tiles_kernel<kTileQ4K, 2>), g, t, 0, s, a, kw);
+    else if (a.quant == PKV_QUANT_Q8_0)
+      hipLaunchKernelGGL((prep_tiles_kernel<kTileQ8, 1>), g, t, 0, s, a, kw);
+    else
+      hipLaunchKernelGGL((prep_tiles_kernel<kTileHalf, 1>), g, t, 0, s, a, kw);
+    PKV_HIP(hipGetLastError());
+    return PKV_OK;
+  }
   hipLaunchKernelGGL(prep_append_kernel, dim3((unsigned)grid), dim3(kPrepThreads), 0, s, a,
                      q_wgs);
   PKV_HIP(hipGetLastError());

@@ -119,6 +119,28 @@ def test_prep_append_bitexact(pk, orc, quant, B, Hkv, D, n_rot):
     same_bytes(g, c)
 
 
+@pytest.mark.parametrize("quant,B,n_rot,ns", [
+    (Q4K, 1, 64, (3, 17, 600)), (Q4K, 2, 64, (2, 9, 700)), (Q4K, 1, 6, (5,)), (Q4K, 1, 256, (33,)),
+    (Q8_0, 1, 64, (1100,)), (F16, 3, 64, (401,)), (BF16, 1, 30, (1030,))])
+def test_prep_append_tiles_bitexact(pk, orc, quant, B, n_rot, ns):
+    """The tiled form (head_dim 256, many rows): ragged tiles of 8 and 16 rows, rotations that
+    end inside a lane's four elements, batches, and K and V alone."""
+    say(f"prep append tiles quant={quant} B={B} n_rot={n_rot} ns={ns}")
+    rng = np.random.default_rng(900 + quant + B + n_rot)
+    cap = sum(ns) + 50
+    L = Layer(pk, orc, 256, n_rot, cap, 17 + quant)
+    g = pk.PreallocatedQuantizedKvCache(B, 2, cap, 256, pk.KvCacheQuantization(quant))
+    c = orc.Cache(quant, B, 2, 256, cap)
+    for n in ns + (50,):
+        q, k, v = rows(rng, (B, n, 16, 256)), rows(rng, (B, n, 2, 256)), rows(rng, (B, n, 2, 256))
+        qp_ref, kp_ref = L.oracle(orc, q, k, c.seq_len)
+        qp = g.append_prep(dev(q) if n != 50 else None, dev(k), dev(v), L.prep)
+        oracle_append(c, kp_ref, v)
+        if n != 50:
+            assert np.array_equal(host(qp).view(np.uint32), qp_ref.view(np.uint32))
+    same_bytes(g, c)
+
+
 @pytest.mark.parametrize("quant,B,n_rot", [(Q4K, 1, 64), (Q4K, 2, 64), (Q4K, 5, 64), (Q4K, 1, 128),
                                            (Q4K, 1, 256), (Q8_0, 1, 64),
                                            (F16, 1, 64)])
