@@ -3,7 +3,7 @@
 // 2657-2680), out[t][o] = sum_i W[o][i] * x[t][i] * sigmoid(g[t][i]), with W a GGUF Q4K,
 // Q5K or Q6K attn_output (self.wo, models/with_tracing.rs:253-300). The per-token form
 // (pkv_oproj.hip) re-reads and re-decodes every weight once per token; here each decoded
-// weight feeds 32 tokens through v_mfma_f32_16x16x32_f16.
+// weight feeds 32 or 64 tokens through v_mfma_f32_16x16x32_f16.
 //
 // Exactness of the fp16 operands:
 //   - activations: a pre-pass gates each token row, scales it by a power of two so that
@@ -23,7 +23,7 @@
 //     both exact, two B operands into the same accumulator, d applied per superblock.
 //
 // Work split: a workgroup of 4 waves owns 256 output rows (64 per wave: four 16-row MFMA
-// tiles) and 32 tokens (two 16-token tiles), over a range of superblocks (split-K when the
+// tiles) and 32 tokens (two 16-token tiles; 64 tokens for many tokens), over a range of superblocks (split-K when the
 // grid would otherwise leave CUs idle; a reduce kernel then sums the partials in split
 // order). Per superblock, the tokens' fp16 fragments (32 KB) and the 256 rows' weight
 // blocks are loaded into registers while the previous superblock computes, and stored to
@@ -522,8 +522,15 @@ int launch_oproj_mfma(const float *attn, const float *gate, const uint8_t *w, in
     if (reinterpret_cast<uintptr_t>(p) % 16 != 0)
       return set_error(PKV_ERR_ARG, "attn, gate and the weights must be 16-byte aligned");
   const int T = batch, N = out_dim, K = in_dim;
-  // tile: 32 tokens x 256 rows per workgroup of 4 waves (32 x 64 per wave)
-  const int tok = 32, rows = 256;
+  // Tile: 32 tokens x 256 rows per workgroup of 4 waves (32 x 64 per wave), and from
+  // kWideTokens tokens on 64 tokens: Q4K and Q5K with 8 waves (two per SIMD, one's decoding
+  // beside the other's MFMAs), Q6K, whose two-plane operands would spill at 256 registers
+  // a wave, with 4 waves of 64 x 64. A decoded weight then feeds twice the tokens; below,
+  // the wide tile leaves CUs idle. us, narrow / wide: Q4K 130 tokens 27.1 / 30.1, 512 47.1 /
+  // 42.3, 4001 296 / 227; Q5K 4001 322 / 245; Q6K 512 65.8 / 61.7, 4001 444 / 377.
+  constexpr int kWideTokens = 384;
+  const bool wide = T >= kWideTokens;
+  const int tok = wide ? 64 : 32, rows = 256;
   const int T_pad = (T + tok - 1) / tok * tok;
   const int KB = K / 32, SB = K / 256;
   const int64_t row_bytes = (int64_t)SB * (w_type == kMQ4K ? 144 : w_type == kMQ5K ? 176 : 210);
@@ -553,11 +560,15 @@ int launch_oproj_mfma(const float *attn, const float *gate, const uint8_t *w, in
             reinterpret_cast<const float *>(base + off_inv), w, row_bytes,
             reinterpret_cast<float *>(base + off_part), out, T, N, KB, SB, per, S, rbs, tbs};
   const dim3 grid((unsigned)(rbs * tbs * S));
-#define PKV_MX(FMT) hipLaunchKernelGGL((oproj_mfma_kernel<FMT, 1, 2, 4>), grid, dim3(256), 0, s, ma)
+#define PKV_MX(FMT, WT, TT)                                                                  \
+  if (wide)                                                                                  \
+    hipLaunchKernelGGL((oproj_mfma_kernel<FMT, WT, TT, 4>), grid, dim3(256 * WT), 0, s, ma); \
+  else                                                                                       \
+    hipLaunchKernelGGL((oproj_mfma_kernel<FMT, 1, 2, 4>), grid, dim3(256), 0, s, ma)
   switch (w_type) {
-    case kMQ4K: PKV_MX(kMQ4K); break;
-    case kMQ5K: PKV_MX(kMQ5K); break;
-    default: PKV_MX(kMQ6K); break;
+    case kMQ4K: PKV_MX(kMQ4K, 2, 2); break;
+    case kMQ5K: PKV_MX(kMQ5K, 2, 2); break;
+    default: PKV_MX(kMQ6K, 1, 4); break;
   }
 #undef PKV_MX
   PKV_HIP(hipGetLastError());
