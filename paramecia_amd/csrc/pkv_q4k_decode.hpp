@@ -955,23 +955,24 @@ __global__ __launch_bounds__(kThreads) void q4k_decode_kernel(
             }
           }
         }
-        if (wg == sg.wg0 && wsub == 0 && n < 8) {  // the combine's copy of the prepared q
-          float *qo = a.q_out + ((int64_t)sg.qi * 16 + 8 * kvu + n) * 256 + 64 * g;
-          if (a.ncomb > 0) {  // read by combiners of this launch, on other XCDs
+        // The combine's copy of the prepared q. One segment: the last workgroup writes it (the
+        // first ones quantize); the in-launch combiners, on other XCDs, read it once the
+        // word below has the launch's parity.
+        const bool publish = (kOne ? wg == nwg_0 - 1 : wg == sg.wg0) && wsub == 0;
+        if (publish && n < 8) {
+          float *qo = a.q_out + ((int64_t)sg.qi * 16 + 8 * kvu) * 256;
+          // (16-byte agent-scope stores: as 64 dword stores per lane they held the
+          // workgroup up: 24.9 us per step at 32768 keys, 19.8 now)
+          const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(qo, 0, 8 * 1024, 0x00020000);
 #pragma unroll
-            for (int st = 0; st < 8; ++st)
+          for (int st = 0; st < 8; ++st)
 #pragma unroll
-              for (int k = 0; k < 8; ++k) store_sc1(qo + 8 * st + k, v[st][k]);
-            // (the wave's word follows below, once every lane's stores are done)
-          } else {
-#pragma unroll
-            for (int st = 0; st < 8; ++st) {
-              *reinterpret_cast<float4 *>(qo + 8 * st) = float4{v[st][0], v[st][1], v[st][2], v[st][3]};
-              *reinterpret_cast<float4 *>(qo + 8 * st + 4) = float4{v[st][4], v[st][5], v[st][6], v[st][7]};
-            }
-          }
+            for (int x = 0; x < 2; ++x)
+              __builtin_amdgcn_raw_buffer_store_b128(
+                  u4{f2u(v[st][4 * x]), f2u(v[st][4 * x + 1]), f2u(v[st][4 * x + 2]), f2u(v[st][4 * x + 3])},
+                  ro, 1024 * n + 256 * g + 32 * st + 16 * x, 0, kSC1);
         }
-        if (a.ncomb > 0 && wg == sg.wg0 && wsub == 0) {  // this wave's q rows are stored
+        if (publish && a.ncomb > 0) {  // this wave's q rows are stored
           asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
           if (lane == 0) store_sc1(a.words + kWordQ + kvu, parity());
         }

@@ -230,3 +230,28 @@ def test_prep_errors_leave_cache_unchanged(pk, orc):
                                     ctypes.c_void_p(kd.data_ptr()), 1, -1)
     assert rc == _lib.ERR_ARG
     assert g.seq_len == 10
+
+
+@pytest.mark.parametrize("S", [32700, 33100])
+def test_prep_decode_full_grid(pk, orc, S):
+    """Around the size from which a prepared decode step merges inside its launch (the
+    combiners wait for the prepared q and the new rows): three steps in a row against the
+    same steps as a prepared append and an attention of its own."""
+    say(f"prep decode full grid S={S}")
+    rng = np.random.default_rng(S)
+    L = Layer(pk, orc, 256, 64, S + 8, 5)
+    k, v = rows(rng, (1, S, 2, 256)), rows(rng, (1, S, 2, 256))
+    g, c = (pk.PreallocatedQuantizedKvCache(1, 2, S + 8, 256, pk.KvCacheQuantization(Q4K)) for _ in range(2))
+    for x in (g, c):
+        x.append_prep(None, dev(k), dev(v), L.prep)
+    for _ in range(3):
+        q, kn, vn = rows(rng, (1, 1, 16, 256)), rows(rng, (1, 1, 2, 256)), rows(rng, (1, 1, 2, 256))
+        got = host(g.append_attend_prep(dev(q), dev(kn), dev(vn), L.prep, 1 / 16))
+        qp = c.append_prep(dev(q), dev(kn), dev(vn), L.prep)
+        ref = host(c.attend(qp, 1 / 16, c.seq_len - 1))
+        np.testing.assert_allclose(got, ref, atol=2e-3, rtol=1e-3)
+        l2 = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+        assert l2 < 2e-5, l2
+        for a, b in zip(g.raw_bytes(), c.raw_bytes()):
+            assert torch.equal(a, b)
+    assert pk.lib().pkv_device_status() == 0
