@@ -64,8 +64,17 @@ def _call(rc: int) -> None:
         raise _ERRORS.get(rc, KvCacheError)(f"[pkv {rc}] {msg}")
 
 
+# torch's own accessors of the current device and its current stream as plain integers:
+# torch.cuda.current_stream() builds a Stream object per call (2.8 us, of the 13 us a short
+# decode step took on the host; 0.3 us this way).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None or _raw_device is None or not torch.cuda.is_initialized():
+        return torch.cuda.current_stream().cuda_stream  # initialises torch's device state
+    return _raw_stream(_raw_device())
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -479,7 +488,7 @@ def gated_o_proj(attn_output: torch.Tensor, gate: Optional[torch.Tensor], wo: to
         raise KvCacheError(f"wo must hold out_dim x in_dim / {blk} blocks of {nbytes} B")
     out = torch.empty(x.shape[:-1] + (out_dim,), dtype=torch.float32, device=x.device)
     _call(lib().pkv_gated_oproj(_ptr(x), _ptr(g), _ptr(wo.contiguous()), w_type, _ptr(out), rows,
-                                in_dim, out_dim, torch.cuda.current_stream().cuda_stream))
+                                in_dim, out_dim, _stream()))
     return out
 
 
@@ -759,8 +768,7 @@ class LinearAttentionState:
         out = torch.empty_like(vv)
         _call(lib().pkv_deltanet_step(_ptr(qq), _ptr(kk), _ptr(vv), _ptr(g), _ptr(bt),
                                       _ptr(rs.ssm_state), _ptr(rs.gate_cumsum_offset), _ptr(out),
-                                      b, H, dv, self.scale, self.eps,
-                                      torch.cuda.current_stream().cuda_stream))
+                                      b, H, dv, self.scale, self.eps, _stream()))
         return out
 
 
@@ -982,8 +990,9 @@ class ModelKvState:
                 ss, cs, gs = cache.layer_caches[i].shapes
                 t = tuple(torch.empty(sh, dtype=torch.float32, device="cuda") for sh in (ss, cs, gs))
                 restored[i] = t
-                targets[i].ssm, targets[i].conv, targets[i].gate_offset = (x.data_ptr() for x in t)
-                targets[i].ssm_cap, targets[i].conv_cap, targets[i].gate_cap = (x.numel() for x in t)
+                target = targets[i]
+                target.ssm, target.conv, target.gate_offset = (x.data_ptr() for x in t)
+                target.ssm_cap, target.conv_cap, target.gate_cap = (x.numel() for x in t)
             targets[i].state_valid = ctypes.cast(ctypes.addressof(valid) + 4 * i,
                                                  ctypes.POINTER(ctypes.c_int))
         ntok = ctypes.c_size_t()
