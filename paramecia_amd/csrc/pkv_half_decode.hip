@@ -5,23 +5,24 @@
 // 2492-2605) for a decode step: every query head reads the keys of KV head h / 8, scores
 // scaled, clamped to +-100, soft-maxed and applied to V.
 //
-// Bound: HBM, 2048 bytes per cached key. No LDS in the loop: a row's halves are MFMA
-// operands as they are. A workgroup of 4 waves owns a range of 32-key blocks of one
-// segment (a cache's batch row, or a sequence); wave w takes KV head w % 2 of every second
-// block, and reads
-//   K as A operands: lane (r, g) takes key kk(r, t), elements 32 s + 8 g .. + 7 (16 bytes);
-//   V as whole 256-byte half rows: lane (n, g) takes elements 128 u + 8 n .. + 7 of keys
-//   8 g .. 8 g + 7, and pairs of keys become B operands with one v_perm per pair and
-//   column: tile 8 u + j holds columns e = 128 u + 8 n + j.
+// Bound: HBM (2048 bytes per cached key) for long caches, the chain of latencies of one
+// 32-key block for short ones, so a block's work is split over the workgroup. A workgroup
+// of 4 waves owns a range of blocks of one KV head of one segment (a cache's batch row, or
+// a sequence). The rows' halves are MFMA operands as they are and go from memory straight
+// into registers, a block ahead:
+//   QK: wave w takes elements 64 w .. 64 w + 63 of all 32 keys (A: lane (r, g) holds 8
+//       elements of key kk(r, t)); the waves' partial scores meet in LDS, one barrier per
+//       block, and every wave then runs the same softmax;
+//   PV: wave w takes columns e = 64 w + 4 n + j: lane (n, g) reads the 8 bytes of columns
+//       4 n .. + 3 of keys 8 g .. 8 g + 7, and pairs of keys become B operands with one
+//       v_perm per pair and column.
 // Keys are permuted inside a block so that the QK result layout is the PV A layout. The
 // new token of a fused step is converted by the first workgroups and joins in the combine
 // (pkv_decode_split.hpp) from its rounded rows.
-// 12290 keys, one layer (25.2 MB): append, general kernel and combine took 160 us; this
-// kernel and its combine take 15.9 us (131073 keys, 268 MB: 56.7 us, 4.7 TB/s). Below 4096
-// keys the 14.4 us are the chain of one block's latencies. Tried: 512 workgroups instead
-// of 256 (32.8 against 22.1 us at 32768 keys: the combine reads twice the partials), V
-// read ahead by a block (16.8 us at 12290).
-//
+// One layer's step (append, attention, combine), us: 12290 keys 160 before, 12.9 now
+// (25.2 MB); 100 keys 7.5, 4096 8.8, 32768 20, 131072 56 (268 MB, 4.8 TB/s). Tried: a wave
+// per block and KV head with its merge in LDS (14.4 at 100 keys, 16.0 at 12290: one wave's
+// serial work), 384 and 512 slots (14.4 and 15.1 at 12290: the combine reads more).
 // Precision: q and the weights p enter as sums of 16-bit parts, accumulated in f32: F16 hi
 // and lo (q scaled by a power of two per row, p by 2^7, so that neither part leaves fp16's
 // range: 22 bits), BF16 three parts (24 bits).
@@ -43,7 +44,7 @@ namespace {
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 
 constexpr int kHdWaves = 4, kHdThreads = 64 * kHdWaves;
-constexpr int kHdTargetWGs = 256;  // partial slots of a full launch
+constexpr int kHdSlots = 256;  // partial slots of a full launch, two workgroups (KV heads) each
 constexpr float kHdLazy = 8.0f;    // log2 headroom of the running max before a rescale
 constexpr float kPBias = 7.0f;     // F16: p is held times 2^7 (at most 2^15 with the headroom)
 
@@ -51,63 +52,60 @@ struct HalfSeg {
   uint8_t *k, *v;  // rows of token 0, KV head 0
   int64_t seq_k;   // keys attended here (a fused step's new key joins in the combine)
   int64_t t_new;   // row the fused step writes
-  int nblk, wg0, nwg;
+  int nblk, wg0, nwg;  // its blocks; its first slot, its slots
 };
 template <int kSegs>
 struct HalfArgs {
-  int64_t rs_t, rs_h;
   int nseg, fused;
-  float sl2;                   // scale * log2(e)
-  const float *q;              // [nseg][16][256]
-  const float *k_new, *v_new;  // [nseg][2][256]
+  float sl2;    // scale * log2(e)
   float *part;                 // [slot][16][256] in tile order
   float2 *ml;                  // [slot][16]
   float *dq;                   // [nseg][4][256]
   HalfSeg seg[kSegs];
 };
 
+// Partial scores of one block: [wave][head][key], rows padded so that the 8 heads' 16-byte
+// reads fall on different banks.
+constexpr int kScoreStride = 36;
 struct HalfSmem {
-  float o[kHdWaves][8][256];
-  float m[kHdWaves][8], l[kHdWaves][8];
+  __attribute__((aligned(16))) float sc[2][kHdWaves][8][kScoreStride];
+  uint32_t bad;
 };
 
 __device__ __forceinline__ float half_value(uint16_t x, bool bf) {
   return bf ? u2f((uint32_t)x << 16) : h2f(x);
 }
 
-// One wave's blocks in f32 products (see the header): lane owns elements 4 lane .. + 3.
-__device__ __forceinline__ void slow_rows(const uint8_t *kbase, const uint8_t *vbase,
-                                          int64_t rs_t, int64_t seq_k, int first, int step,
-                                          int last, const float *q, float sl2, bool bf, int lane,
-                                          float (*o)[256], float *mo, float *lo) {
-  for (int h = 0; h < 8; ++h) {
+// Heads h0 and h0 + 1 of a workgroup's blocks [b0, b1) in f32 products (see the header),
+// stored as its partial: lane owns elements 4 lane .. + 3.
+__device__ __forceinline__ void slow_heads(const uint8_t *kbase, const uint8_t *vbase,
+                                           int64_t rs_t, int64_t seq_k, int b0, int b1,
+                                           const float *q, int h0, float sl2, bool bf, int lane,
+                                           float *part, float2 *ml) {
+  for (int h = h0; h < h0 + 2; ++h) {
     const float4 q4 = reinterpret_cast<const float4 *>(q + h * 256)[lane];
     float m = -INFINITY, l = 0.0f, acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int b = first; b < last; b += step) {
-      const int64_t k1 = (int64_t)(b + 1) * kBlk < seq_k ? (int64_t)(b + 1) * kBlk : seq_k;
-      for (int64_t j = (int64_t)b * kBlk; j < k1; ++j) {
-        const uint2 kw = *reinterpret_cast<const uint2 *>(kbase + j * rs_t + 8 * lane);
-        const uint2 vw = *reinterpret_cast<const uint2 *>(vbase + j * rs_t + 8 * lane);
-        float part = q4.x * half_value((uint16_t)kw.x, bf);
-        part += q4.y * half_value((uint16_t)(kw.x >> 16), bf);
-        part += q4.z * half_value((uint16_t)kw.y, bf);
-        part += q4.w * half_value((uint16_t)(kw.y >> 16), bf);
-        const float s = fminf(fmaxf(wave_sum(part) * sl2, -kClampL2), kClampL2);
-        const float mn = fmaxf(m, s);
-        const float c = __builtin_amdgcn_exp2f(m - mn), p = __builtin_amdgcn_exp2f(s - mn);
-        l = l * c + p;
-        acc[0] = acc[0] * c + p * half_value((uint16_t)vw.x, bf);
-        acc[1] = acc[1] * c + p * half_value((uint16_t)(vw.x >> 16), bf);
-        acc[2] = acc[2] * c + p * half_value((uint16_t)vw.y, bf);
-        acc[3] = acc[3] * c + p * half_value((uint16_t)(vw.y >> 16), bf);
-        m = mn;
-      }
+    const int64_t k1 = (int64_t)b1 * kBlk < seq_k ? (int64_t)b1 * kBlk : seq_k;
+    for (int64_t j = (int64_t)b0 * kBlk; j < k1; ++j) {
+      const uint2 kw = *reinterpret_cast<const uint2 *>(kbase + j * rs_t + 8 * lane);
+      const uint2 vw = *reinterpret_cast<const uint2 *>(vbase + j * rs_t + 8 * lane);
+      float dot = q4.x * half_value((uint16_t)kw.x, bf);
+      dot += q4.y * half_value((uint16_t)(kw.x >> 16), bf);
+      dot += q4.z * half_value((uint16_t)kw.y, bf);
+      dot += q4.w * half_value((uint16_t)(kw.y >> 16), bf);
+      const float s = fminf(fmaxf(wave_sum(dot) * sl2, -kClampL2), kClampL2);
+      const float mn = fmaxf(m, s);
+      const float c = __builtin_amdgcn_exp2f(m - mn), p = __builtin_amdgcn_exp2f(s - mn);
+      l = l * c + p;
+      acc[0] = acc[0] * c + p * half_value((uint16_t)vw.x, bf);
+      acc[1] = acc[1] * c + p * half_value((uint16_t)(vw.x >> 16), bf);
+      acc[2] = acc[2] * c + p * half_value((uint16_t)vw.y, bf);
+      acc[3] = acc[3] * c + p * half_value((uint16_t)(vw.y >> 16), bf);
+      m = mn;
     }
-    *reinterpret_cast<float4 *>(&o[h][4 * lane]) = float4{acc[0], acc[1], acc[2], acc[3]};
-    if (lane == 0) {
-      mo[h] = m;
-      lo[h] = l;
-    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) part[h * kPartRow + tile_index(4 * lane + k)] = acc[k];
+    if (lane == 0) ml[h] = float2{m, l};
   }
 }
 
@@ -144,81 +142,110 @@ __device__ __forceinline__ f4 half_mfma(u4 a, u4 b, f4 c) {
   else
     return mfma32(__builtin_bit_cast(h8, a), __builtin_bit_cast(h8, b), c);
 }
-__device__ __forceinline__ u4 row16(__amdgpu_buffer_rsrc_t r, uint32_t off, int imm) {
-  return __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(r, off + imm, 0, 0));
+template <typename T>
+__device__ __forceinline__ T row_load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  if constexpr (sizeof(T) == 16)
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  else
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+}
+// LDS written before is visible to the workgroup after; loads from memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// The leading scalar arguments (segment 0's rows and keys, q, the new rows, rs_t | rs_h <<
+// 24, the workgroups) are preloaded into SGPRs, so a one-segment launch's first loads wait
+// for no kernel-argument fetch. knew_0 / vnew_0 are q_0 in an attention without an append.
 template <bool kBf, int kSegs>
-__global__ __launch_bounds__(kHdThreads) void half_decode_kernel(HalfArgs<kSegs> a) {
+__global__ __launch_bounds__(kHdThreads) void half_decode_kernel(
+    const uint8_t *k_0, const uint8_t *v_0, const float *q_0, const float *knew_0,
+    const float *vnew_0, uint64_t strides, int seq_k0, int nwg_0, HalfArgs<kSegs> a) {
   __shared__ HalfSmem sm;
   const int tid = threadIdx.x, lane = tid & 63, n = lane & 15, g = lane >> 4;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), kv = wave & 1, sub = wave >> 1;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int slot = (int)blockIdx.x >> 1, kv = (int)blockIdx.x & 1;
   int s = 0;
   if constexpr (kSegs > 1)
-    while (s + 1 < a.nseg && a.seg[s + 1].wg0 <= (int)blockIdx.x) ++s;
-  const HalfSeg sg = a.seg[s];
+    while (s + 1 < a.nseg && a.seg[s + 1].wg0 <= slot) ++s;
+  HalfSeg sg;
+  if constexpr (kSegs == 1) {
+    sg.k = const_cast<uint8_t *>(k_0);
+    sg.v = const_cast<uint8_t *>(v_0);
+    sg.seq_k = seq_k0;
+    sg.nblk = (seq_k0 + kBlk - 1) / kBlk;
+    sg.wg0 = 0;
+    sg.nwg = nwg_0;
+  } else {
+    sg = a.seg[s];
+  }
+  const int64_t rs_h = (int64_t)(strides >> 24);
   // blocks [b0, b1) of the segment
-  const int w = (int)blockIdx.x - sg.wg0, bq = sg.nblk / sg.nwg, br = sg.nblk % sg.nwg;
+  const int w = slot - sg.wg0, bq = sg.nblk / sg.nwg, br = sg.nblk % sg.nwg;
   const int b0 = w * bq + (w < br ? w : br), b1 = b0 + bq + (w < br ? 1 : 0);
-  const uint32_t rs_t = (uint32_t)a.rs_t;
-  const uint8_t *kbase = sg.k + kv * a.rs_h, *vbase = sg.v + kv * a.rs_h;
+  const uint32_t rs_t = (uint32_t)(strides & 0xFFFFFFu);
+  const uint8_t *kbase = sg.k + kv * rs_h, *vbase = sg.v + kv * rs_h;
   const int last = (int)sg.seq_k - 1;  // loads past it read the last row again (masked)
   const uint32_t span = sg.seq_k > 0 ? (uint32_t)last * rs_t + 512u : 0u;
   const __amdgpu_buffer_rsrc_t rk =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(kbase), 0, span, 0x00020000);
   const __amdgpu_buffer_rsrc_t rv =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(vbase), 0, span, 0x00020000);
-  u4 kw[2][8], vw[8][2];
+  u4 kw[2][2];
+  uint2 vw[8];
   auto load_k = [&](int b) {
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       const int key = b * kBlk + 8 * (n >> 2) + 4 * t + (n & 3);
-      const uint32_t off = (uint32_t)(key < last ? key : last) * rs_t + 16u * g;
+      const uint32_t off = (uint32_t)(key < last ? key : last) * rs_t + 128u * wave + 16u * g;
 #pragma unroll
-      for (int st = 0; st < 8; ++st) kw[t][st] = row16(rk, off, 64 * st);
+      for (int st = 0; st < 2; ++st) kw[t][st] = row_load<u4>(rk, off + 64 * st);
     }
   };
   auto load_v = [&](int b) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       const int key = b * kBlk + 8 * g + k;
-      const uint32_t off = (uint32_t)(key < last ? key : last) * rs_t + 16u * n;
-      vw[k][0] = row16(rv, off, 0);
-      vw[k][1] = row16(rv, off, 256);
+      vw[k] = row_load<uint2>(rv, (uint32_t)(key < last ? key : last) * rs_t + 128u * wave + 8u * n);
     }
   };
-  const int first = b0 + sub;
-  const float *qseg = a.q + ((int64_t)s * 16 + 8 * kv) * 256;
-  // q operands: lane (n, g) holds elements 32 st + 8 g .. + 7 of head n % 8
-  float4 qv[8][2];
+  const float *qseg = q_0 + ((int64_t)s * 16 + 8 * kv) * 256;
+  // q: lane (n, g) holds elements 64 wave + 32 st + 8 g .. + 7 of head n % 8
+  float4 qv[2][2];
 #pragma unroll
-  for (int st = 0; st < 8; ++st)
+  for (int st = 0; st < 2; ++st)
 #pragma unroll
     for (int x = 0; x < 2; ++x)
-      qv[st][x] = *reinterpret_cast<const float4 *>(qseg + (n & 7) * 256 + 32 * st + 8 * g + 4 * x);
-  if (first < b1) {
-    load_k(first);
+      qv[st][x] = *reinterpret_cast<const float4 *>(qseg + (n & 7) * 256 + 64 * wave + 32 * st + 8 * g + 4 * x);
+  // (every workgroup loads a new row's element, so that the load sits in no branch and is
+  // waited for where it is used)
+  const int new0 = (int)blockIdx.x < 4 * a.nseg ? (int)blockIdx.x : 0;
+  float xn = ((new0 & 2) ? vnew_0 : knew_0)[((int64_t)(new0 >> 2) * 2 + (new0 & 1)) * 256 + tid];
+  if (b0 < b1) {
+    load_k(b0);
+    load_v(b0);
   }
+  if (tid == 0) sm.bad = 0u;
 
   // Fused step: row 4 i + 2 p + kv (segment i, K (p = 0) or V) is converted and stored
   if (a.fused) {
     for (int row = blockIdx.x; row < 4 * a.nseg; row += gridDim.x) {
       const int i = row >> 2, p = (row >> 1) & 1, h = row & 1;
-      const float x = (p ? a.v_new : a.k_new)[((int64_t)i * 2 + h) * 256 + tid];
-      const uint16_t y = kBf ? f32_to_bf16(x) : f32_to_f16(x);
+      if (row != (int)blockIdx.x) xn = (p ? vnew_0 : knew_0)[((int64_t)i * 2 + h) * 256 + tid];
+      const uint16_t y = kBf ? f32_to_bf16(xn) : f32_to_f16(xn);
       const HalfSeg &r = a.seg[kSegs > 1 ? i : 0];
-      reinterpret_cast<uint16_t *>((p ? r.v : r.k) + r.t_new * a.rs_t + h * a.rs_h)[tid] = y;
+      reinterpret_cast<uint16_t *>((p ? r.v : r.k) + r.t_new * rs_t + h * rs_h)[tid] = y;
       a.dq[(int64_t)row * 256 + tid] = half_value(y, kBf);
     }
   }
 
-  u4 qb[8], qb2[8];
-  float cs = a.sl2;  // a score is its MFMA result * cs, in log2 units
-  float f = 1.0f;
-  if constexpr (!kBf) {  // q to [2^14, 2^15)
+  float f = 1.0f, back = 1.0f;  // q enters times f, a partial score leaves times 1 / f
+  if constexpr (!kBf) {  // the wave's elements of a row to [2^14, 2^15)
     float mx = 0.0f;
 #pragma unroll
-    for (int st = 0; st < 8; ++st)
+    for (int st = 0; st < 2; ++st)
 #pragma unroll
       for (int x = 0; x < 2; ++x)
         mx = fmaxf(mx, fmaxf(fmaxf(fabsf(qv[st][x].x), fabsf(qv[st][x].y)),
@@ -227,10 +254,11 @@ __global__ __launch_bounds__(kHdThreads) void half_decode_kernel(HalfArgs<kSegs>
     int e = (int)(f2u(mx) >> 23) - 127;
     e = e < -100 ? -100 : e > 100 ? 100 : e;
     f = __builtin_ldexpf(1.0f, 14 - e);
-    cs = a.sl2 * __builtin_ldexpf(1.0f, e - 14);
+    back = __builtin_ldexpf(1.0f, e - 14);
   }
+  u4 qb[2], qb2[2];
 #pragma unroll
-  for (int st = 0; st < 8; ++st) {
+  for (int st = 0; st < 2; ++st) {
     uint32_t w1[4], w2[4];
 #pragma unroll
     for (int x = 0; x < 2; ++x) {
@@ -242,41 +270,60 @@ __global__ __launch_bounds__(kHdThreads) void half_decode_kernel(HalfArgs<kSegs>
   }
 
   const f4 zero = {0.f, 0.f, 0.f, 0.f};
-  f4 acc[16];
+  f4 acc[4];
 #pragma unroll
-  for (int T = 0; T < 16; ++T) acc[T] = zero;
-  // Scores and the running max stay in MFMA units; the scale enters the exponents as one
+  for (int j = 0; j < 4; ++j) acc[j] = zero;
+  // Scores and the running max stay in q . k units; the scale enters the exponents as one
   // fma (rounding a score of tens of log2 units instead cost 2-4 times the error where a
   // few keys dominate). nm: log2 of the weights' common factor.
   constexpr float kBias = kBf ? 0.0f : kPBias;
-  const float clamp = kClampL2 / cs, lazy = kHdLazy / cs;
+  const float cs = a.sl2, clamp = kClampL2 / cs, lazy = kHdLazy / cs;
   float m_run = -INFINITY, nm = INFINITY, lsum = 0.0f;
   bool bad = false;
-  for (int b = first; b < b1; b += 2) {
-    load_v(b);
-    // ---- scores of keys 8 g + 4 t + i, head n % 8 (hi columns n < 8, lo columns n >= 8)
-    float sc8[8];
+  for (int b = b0; b < b1; ++b) {
+    // ---- the wave's part of the scores: keys 8 g + 4 t + i, head n % 8 (hi columns n < 8,
+    // lo columns n >= 8)
+    float(*sc)[8][kScoreStride] = sm.sc[(b - b0) & 1];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-      f4 c0 = zero, c1 = zero;
+      f4 c = zero;
 #pragma unroll
-      for (int st = 0; st < 8; st += 2) {
-        c0 = half_mfma<kBf>(kw[t][st], qb[st], c0);
-        c1 = half_mfma<kBf>(kw[t][st + 1], qb[st + 1], c1);
-        if constexpr (kBf) {
-          c0 = half_mfma<kBf>(kw[t][st], qb2[st], c0);
-          c1 = half_mfma<kBf>(kw[t][st + 1], qb2[st + 1], c1);
-        }
+      for (int st = 0; st < 2; ++st) {
+        c = half_mfma<kBf>(kw[t][st], qb[st], c);
+        if constexpr (kBf) c = half_mfma<kBf>(kw[t][st], qb2[st], c);
       }
+      float4 r;
+      r.x = (c[0] + ror8(c[0])) * back;
+      r.y = (c[1] + ror8(c[1])) * back;
+      r.z = (c[2] + ror8(c[2])) * back;
+      r.w = (c[3] + ror8(c[3])) * back;
+      if (n < 8) *reinterpret_cast<float4 *>(&sc[wave][n][8 * g + 4 * t]) = r;
+    }
+    if (b + 1 < b1) load_k(b + 1);
+    // (the scores alternate between two buffers: a wave that is a block ahead writes the
+    // other one)
+    lds_barrier();
+    float sc8[8];
+    {
+      float4 pw[kHdWaves][2];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float part = c0[i] + c1[i];
-        const float sum = part + ror8(part);
-        bad |= !(fabsf(sum) < INFINITY);
-        sc8[4 * t + i] = __builtin_amdgcn_fmed3f(sum, -clamp, clamp);
+      for (int x = 0; x < kHdWaves; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+          pw[x][y] = *reinterpret_cast<const float4 *>(&sc[x][n & 7][8 * g + 4 * y]);
+#pragma unroll
+      for (int y = 0; y < 2; ++y) {
+        sc8[4 * y] = (pw[0][y].x + pw[1][y].x) + (pw[2][y].x + pw[3][y].x);
+        sc8[4 * y + 1] = (pw[0][y].y + pw[1][y].y) + (pw[2][y].y + pw[3][y].y);
+        sc8[4 * y + 2] = (pw[0][y].z + pw[1][y].z) + (pw[2][y].z + pw[3][y].z);
+        sc8[4 * y + 3] = (pw[0][y].w + pw[1][y].w) + (pw[2][y].w + pw[3][y].w);
       }
     }
-    if (b + 2 < b1) load_k(b + 2);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      bad |= !(fabsf(sc8[k]) < INFINITY);
+      sc8[k] = __builtin_amdgcn_fmed3f(sc8[k], -clamp, clamp);
+    }
     const int nvalid = (int)sg.seq_k - b * kBlk;
     if (nvalid < kBlk) {
 #pragma unroll
@@ -301,9 +348,9 @@ __global__ __launch_bounds__(kHdThreads) void half_decode_kernel(HalfArgs<kSegs>
 #pragma unroll
       for (int i = 0; i < 4; ++i) ai[i] = __shfl(alpha, 4 * (g & 1) + i);
 #pragma unroll
-      for (int T = 0; T < 16; ++T)
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) acc[T][i] *= ai[i];
+        for (int i = 0; i < 4; ++i) acc[j][i] *= ai[i];
     }
     float p[8];
 #pragma unroll
@@ -319,76 +366,59 @@ __global__ __launch_bounds__(kHdThreads) void half_decode_kernel(HalfArgs<kSegs>
       A = u4{w1[0], w1[1], w1[2], w1[3]};
       A2 = u4{w2[0], w2[1], w2[2], w2[3]};
     }
-    // ---- PV: tile 8 u + j, column n: e = 128 u + 8 n + j
+    // ---- PV: tile j, column n: e = 64 wave + 4 n + j
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
+      uint32_t bw[4];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;
-        uint32_t bw[4];
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          bw[k] = __builtin_amdgcn_perm(vw[2 * k + 1][u][j >> 1], vw[2 * k][u][j >> 1], sel);
-        const u4 B = {bw[0], bw[1], bw[2], bw[3]};
-        acc[8 * u + j] = half_mfma<kBf>(A, B, acc[8 * u + j]);
-        if constexpr (kBf) acc[8 * u + j] = half_mfma<kBf>(A2, B, acc[8 * u + j]);
-      }
+      for (int k = 0; k < 4; ++k)
+        bw[k] = j < 2 ? __builtin_amdgcn_perm(vw[2 * k + 1].x, vw[2 * k].x, sel)
+                      : __builtin_amdgcn_perm(vw[2 * k + 1].y, vw[2 * k].y, sel);
+      const u4 B = {bw[0], bw[1], bw[2], bw[3]};
+      acc[j] = half_mfma<kBf>(A, B, acc[j]);
+      if constexpr (kBf) acc[j] = half_mfma<kBf>(A2, B, acc[j]);
+    }
+    if (b + 1 < b1) load_v(b + 1);
   }
 
-  // ---- this wave's rows into LDS: rows h and h + 8 summed (lanes 0-31 keep the columns of
-  // u = 0, lanes 32-63 those of u = 1), heads 4 (g & 1) + i
+  // ---- the partial: rows h and h + 8 summed (lanes 0-31 keep tiles 0 and 1, lanes 32-63
+  // tiles 2 and 3), heads 4 (g & 1) + i, in tile order (tile_index of the columns)
   lsum += __shfl_xor(lsum, 16);
   lsum += __shfl_xor(lsum, 32);
-  const int gr = g & 1, u = g >> 1;
+  float *part = a.part + ((int64_t)slot * 16 + 8 * kv) * kPartRow;
+  float2 *ml = a.ml + (int64_t)slot * 16 + 8 * kv;
+  float r[2][4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float r[8];
+  for (int y = 0; y < 2; ++y)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      r[j] = pair_sum32(acc[j][i], acc[8 + j][i]);
-      bad |= !(fabsf(r[j]) < INFINITY);
+    for (int i = 0; i < 4; ++i) {
+      r[y][i] = pair_sum32(acc[y][i], acc[y + 2][i]);
+      bad |= !(fabsf(r[y][i]) < INFINITY);
     }
-    float *o = &sm.o[wave][4 * gr + i][128 * u + 8 * n];
-    reinterpret_cast<float4 *>(o)[0] = float4{r[0], r[1], r[2], r[3]};
-    reinterpret_cast<float4 *>(o)[1] = float4{r[4], r[5], r[6], r[7]};
+  if (bad) sm.bad = 1u;
+  lds_barrier();
+  if (sm.bad != 0u) {
+    slow_heads(kbase, vbase, rs_t, sg.seq_k, b0, b1, qseg, 2 * wave, a.sl2, kBf, lane, part, ml);
+    return;
   }
-  if (lane < 8) {
-    sm.m[wave][n] = -nm;
-    sm.l[wave][n] = lsum;
-  }
-  if (__any(bad))
-    slow_rows(kbase, vbase, a.rs_t, sg.seq_k, first, 2, b1, qseg, a.sl2, kBf, lane, sm.o[wave],
-              sm.m[wave], sm.l[wave]);
-  __syncthreads();
-  // ---- the two waves of each KV head merged into the workgroup's partial, in tile order
-  const int e = tile_e(tid >> 4, tid & 15);
 #pragma unroll
-  for (int h = 0; h < 16; ++h) {
-    const int w0 = h >> 3, w1 = w0 + 2, r = h & 7;
-    const float m0 = sm.m[w0][r], m1 = sm.m[w1][r], M = fmaxf(m0, m1);
-    float v = 0.0f, L = 0.0f;
-    if (m0 != -INFINITY) {
-      const float c = __builtin_amdgcn_exp2f(m0 - M);
-      v = sm.o[w0][r][e] * c;
-      L = sm.l[w0][r] * c;
-    }
-    if (m1 != -INFINITY) {
-      const float c = __builtin_amdgcn_exp2f(m1 - M);
-      v += sm.o[w1][r][e] * c;
-      L += sm.l[w1][r] * c;
-    }
-    const int64_t slot = (int64_t)blockIdx.x * 16 + h;
-    __builtin_nontemporal_store(v, a.part + slot * kPartRow + tid);
-    if (tid == 0) a.ml[slot] = float2{M, L};
+  for (int y = 0; y < 2; ++y) {
+    const int at = tile_index(64 * wave + 4 * n + 2 * (g >> 1) + y);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      __builtin_nontemporal_store(r[y][i], part + (4 * (g & 1) + i) * kPartRow + at);
   }
+  if (wave == 0 && lane < 8) ml[n] = float2{-nm, lsum};
 }
 
 // Plan and launch the decode and the combine over n <= kMaxSegs segments. Every segment
-// gets workgroups in proportion to its blocks, at most one per two blocks (a block per
-// wave pair) and kHdTargetWGs in all (and at least one each).
+// gets slots in proportion to its blocks, at most one per block and about kHdSlots in all
+// (and at least one each).
 int launch_half_segments(int quant, const DecodeSegIn *in, int n, const float *q,
                          const float *k_new, const float *v_new, float *out, int64_t rs_t,
                          int64_t rs_h, float scale, Workspace &ws, hipStream_t s) {
+  if (!decode_head_stride_fits(rs_h)) return PKV_ERR_UNSUPPORTED;
   HalfArgs<kMaxSegs> d;
   CombineArgs c;
   const bool fused = k_new != nullptr, bf = quant == PKV_QUANT_BF16;
@@ -405,8 +435,8 @@ int launch_half_segments(int quant, const DecodeSegIn *in, int n, const float *q
   int slots = 0;
   for (int i = 0; i < n; ++i) {
     HalfSeg &g = d.seg[i];
-    int64_t share = total > 0 ? (g.nblk * (int64_t)kHdTargetWGs + total / 2) / total : 1;
-    if (share > (g.nblk + 1) / 2) share = (g.nblk + 1) / 2;
+    int64_t share = total > 0 ? (g.nblk * (int64_t)kHdSlots + total / 2) / total : 1;
+    if (share > g.nblk) share = g.nblk;
     g.nwg = share < 1 ? 1 : (int)share;
     g.wg0 = slots;
     c.wg0[i] = slots;
@@ -416,40 +446,37 @@ int launch_half_segments(int quant, const DecodeSegIn *in, int n, const float *q
   const size_t part_floats = (size_t)slots * 16 * kPartRow, ml_floats = (size_t)slots * 16 * 2;
   const int rc = ws.reserve((part_floats + ml_floats + (size_t)n * 4 * 256) * sizeof(float));
   if (rc) return rc;
-  d.rs_t = rs_t;
-  d.rs_h = rs_h;
   d.nseg = n;
   d.fused = fused;
   d.sl2 = scale * kLog2e;
-  d.q = q;
-  d.k_new = k_new;
-  d.v_new = v_new;
   d.part = static_cast<float *>(ws.ptr);
   d.ml = reinterpret_cast<float2 *>(d.part + part_floats);
   d.dq = d.part + part_floats + ml_floats;
-  const dim3 grid((unsigned)slots), block(kHdThreads);
+  const dim3 grid((unsigned)(2 * slots)), block(kHdThreads);
+  const float *kn = fused ? k_new : q, *vn = fused ? v_new : q;
+  const uint64_t st = decode_strides(rs_t, rs_h);
+  const int seq0 = (int)d.seg[0].seq_k, nwg0 = d.seg[0].nwg;
   if (n == 1) {
     HalfArgs<1> d1;
-    d1.rs_t = d.rs_t;
-    d1.rs_h = d.rs_h;
     d1.nseg = 1;
     d1.fused = d.fused;
     d1.sl2 = d.sl2;
-    d1.q = q;
-    d1.k_new = k_new;
-    d1.v_new = v_new;
     d1.part = d.part;
     d1.ml = d.ml;
     d1.dq = d.dq;
     d1.seg[0] = d.seg[0];
     if (bf)
-      hipLaunchKernelGGL((half_decode_kernel<true, 1>), grid, block, 0, s, d1);
+      hipLaunchKernelGGL((half_decode_kernel<true, 1>), grid, block, 0, s, d.seg[0].k, d.seg[0].v, q,
+                         kn, vn, st, seq0, nwg0, d1);
     else
-      hipLaunchKernelGGL((half_decode_kernel<false, 1>), grid, block, 0, s, d1);
+      hipLaunchKernelGGL((half_decode_kernel<false, 1>), grid, block, 0, s, d.seg[0].k, d.seg[0].v, q,
+                         kn, vn, st, seq0, nwg0, d1);
   } else if (bf) {
-    hipLaunchKernelGGL((half_decode_kernel<true, kMaxSegs>), grid, block, 0, s, d);
+    hipLaunchKernelGGL((half_decode_kernel<true, kMaxSegs>), grid, block, 0, s, d.seg[0].k,
+                       d.seg[0].v, q, kn, vn, st, seq0, nwg0, d);
   } else {
-    hipLaunchKernelGGL((half_decode_kernel<false, kMaxSegs>), grid, block, 0, s, d);
+    hipLaunchKernelGGL((half_decode_kernel<false, kMaxSegs>), grid, block, 0, s, d.seg[0].k,
+                       d.seg[0].v, q, kn, vn, st, seq0, nwg0, d);
   }
   PKV_HIP(hipGetLastError());
   c.part = d.part;
