@@ -14,7 +14,6 @@
 #include "pkv_internal.hpp"
 #include "pkv_scalar.hpp"
 #include "pkv_q4k_fit.hpp"
-#include "pkv_q4k_lanes.hpp"
 
 namespace pkv {
 namespace {
@@ -82,7 +81,7 @@ __global__ __launch_bounds__(256) void q4k_append_kernel(AppendArgs a, int64_t u
   float x[E];
   const int e0 = sb * 256 + 32 * j + s * E;
   const float *src = a.src[p];
-  if ((a.head_dim & 3) == 0 && e0 + E <= a.head_dim) {
+  if ((a.head_dim & 3) == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0 && e0 + E <= a.head_dim) {
     const float4 *s4 = reinterpret_cast<const float4 *>(
         src + (((int64_t)b * a.heads + h) * a.n + t) * a.head_dim + e0);
 #pragma unroll
@@ -101,59 +100,89 @@ __global__ __launch_bounds__(256) void q4k_append_kernel(AppendArgs a, int64_t u
   q4k_quantize_group<kL>(x, r, row_ptr(a, p, t, b, h) + (int64_t)sb * 144, active);
 }
 
-// One workgroup per (tensor, token, batch, head, superblock); for appends of a few rows.
-__global__ __launch_bounds__(256) void q4k_append_small_kernel(AppendArgs a, int nsb) {
-  __shared__ Q4kScratch scr;
-  int64_t u = blockIdx.x;
-  const int sb = (int)(u % nsb);
-  u /= nsb;
-  const int h = (int)(u % a.heads);
-  u /= a.heads;
-  const int b = (int)(u % a.batch);
-  u /= a.batch;
-  const int64_t t = u % a.n;
-  const int p = (int)(u / a.n);
-  const float x = load_elem(a.src[p], a, t, b, h, sb * 256 + (int)threadIdx.x);
-  uint8_t *blk = row_ptr(a, p, t, b, h) + (int64_t)sb * 144;
-  q4k_quantize_superblock_lanes(x, blk, &scr, (int)threadIdx.x);
-}
-
-// Q8_0 (BlockQ8_0::from_float): one lane per 32-element block.
-__global__ __launch_bounds__(256) void q8_0_append_kernel(AppendArgs a, int64_t units_per_tensor,
-                                                          int nblk) {
-  const int64_t unit = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (unit >= 2 * units_per_tensor) return;
-  const int p = (int)(unit / units_per_tensor);
-  int64_t u = unit % units_per_tensor;
-  const int blk = (int)(u % nblk);
-  u /= nblk;
-  const int h = (int)(u % a.heads);
-  u /= a.heads;
-  const int b = (int)(u % a.batch);
-  const int64_t t = u / a.batch;
-  float x[32];
+// Four elements of a row per lane: 16-byte loads where kWide (head_dim a multiple of 4, K
+// and V 16-byte aligned), else one by one. U counts lanes: 32 bits but for appends of 2^31
+// lanes and more. A lane's tensor p, row (t, b, h) and elements e .. e + 3; false past the end.
+struct Quad {
+  float x[4];
+  int p, b, h, e;
+  int64_t t;
+};
+template <bool kWide, typename U>
+__device__ __forceinline__ bool load_quad(const AppendArgs &a, U quads_per_tensor, Quad &q) {
+  const U i = (U)blockIdx.x * 256 + threadIdx.x;
+  if (i >= 2 * quads_per_tensor) return false;
+  q.p = i >= quads_per_tensor;
+  const U u = q.p ? i - quads_per_tensor : i;
+  const U per_row = (U)a.padded >> 2, r = u / per_row;
+  q.e = (int)(u - r * per_row) * 4;
+  const U rh = r / (U)a.heads, t = rh / (U)a.batch;
+  q.h = (int)(r - rh * (U)a.heads);
+  q.t = (int64_t)t;
+  q.b = (int)(rh - t * (U)a.batch);
+  const float *src = a.src[q.p];
+  if constexpr (kWide) {
+    float4 f = {0.f, 0.f, 0.f, 0.f};
+    if (q.e < a.head_dim)
+      f = *reinterpret_cast<const float4 *>(
+          src + (((int64_t)q.b * a.heads + q.h) * a.n + q.t) * a.head_dim + q.e);
+    q.x[0] = f.x;
+    q.x[1] = f.y;
+    q.x[2] = f.z;
+    q.x[3] = f.w;
+  } else {
 #pragma unroll
-  for (int i = 0; i < 32; ++i) x[i] = load_elem(a.src[p], a, t, b, h, blk * 32 + i);
-  float amax = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 32; ++i) amax = fmax_rs(amax, __builtin_fabsf(x[i]));
-  const float d = amax / 127.0f;
-  const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
-  uint16_t w[17];
-  w[0] = f32_to_f16(d);
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    uint32_t q0 = (uint8_t)rs_as_i8(__builtin_roundf(x[2 * i] * id));
-    uint32_t q1 = (uint8_t)rs_as_i8(__builtin_roundf(x[2 * i + 1] * id));
-    w[1 + i] = (uint16_t)(q0 | (q1 << 8));
+    for (int k = 0; k < 4; ++k) q.x[k] = load_elem(src, a, q.t, q.b, q.h, q.e + k);
   }
-  uint16_t *dst =
-      reinterpret_cast<uint16_t *>(row_ptr(a, p, t, b, h) + (int64_t)blk * 34);
-#pragma unroll
-  for (int i = 0; i < 17; ++i) dst[i] = w[i];
+  return true;
 }
 
-// F16 / BF16 rows: element-wise round-to-nearest-even conversion.
+// Q8_0 (BlockQ8_0::from_float): 8 lanes per 32-element block, four elements each, so that a
+// wave reads 1 KB and writes 272 bytes in a row. The block's largest |x| is exact in any
+// order (NaN dropped, as f32::max does). One lane per block, with 32 scalar loads and 17
+// 2-byte stores, took 11.0 us for 512 tokens of the model's shape (2.7 MB), this form 3.3 us.
+template <bool kWide, typename U>
+__global__ __launch_bounds__(256) void q8_0_append_kernel(AppendArgs a, U quads_per_tensor) {
+  Quad q;
+  if (!load_quad<kWide, U>(a, quads_per_tensor, q)) return;
+  int32_t key = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int32_t v = (q.x[k] != q.x[k]) ? 0 : (int32_t)(f2u(q.x[k]) & 0x7FFFFFFFu);
+    key = v > key ? v : key;
+  }
+#pragma unroll
+  for (int o = 1; o < 8; o <<= 1) {
+    const int32_t v = __shfl_xor(key, o, 8);
+    key = v > key ? v : key;
+  }
+  const float d = u2f((uint32_t)key) / 127.0f;
+  const float id = (d != 0.0f) ? 1.0f / d : 0.0f;
+  uint32_t w = 0u;
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+    w |= (uint32_t)(uint8_t)rs_as_i8(__builtin_roundf(q.x[k] * id)) << (8 * k);
+  uint8_t *blk = row_ptr(a, q.p, q.t, q.b, q.h) + (q.e >> 5) * 34;
+  uint16_t *o = reinterpret_cast<uint16_t *>(blk + 2 + (q.e & 31));
+  o[0] = (uint16_t)w;
+  o[1] = (uint16_t)(w >> 16);
+  if ((q.e & 31) == 0) *reinterpret_cast<uint16_t *>(blk) = f32_to_f16(d);
+}
+
+// F16 / BF16 rows: round-to-nearest-even conversion, four elements a lane (4096 tokens of
+// the model's shape 20.9 us one by one, 9.5 now). Rows of a head_dim that is no multiple
+// of 4 go element by element.
+template <bool BF, bool kWide>
+__global__ __launch_bounds__(256) void half_append_quads_kernel(AppendArgs a,
+                                                                uint32_t quads_per_tensor) {
+  Quad q;
+  if (!load_quad<kWide, uint32_t>(a, quads_per_tensor, q)) return;
+  uint32_t y[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) y[k] = BF ? f32_to_bf16(q.x[k]) : f32_to_f16(q.x[k]);
+  *reinterpret_cast<uint2 *>(row_ptr(a, q.p, q.t, q.b, q.h) + 2 * q.e) =
+      uint2{y[0] | (y[1] << 16), y[2] | (y[3] << 16)};
+}
 template <bool BF>
 __global__ __launch_bounds__(256) void half_append_kernel(AppendArgs a, int64_t elems_per_tensor) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -273,14 +302,14 @@ static int launch_append_args(int quant, AppendArgs &a, hipStream_t s) {
   const int batch = a.batch, heads = a.heads;
   const int64_t n = a.n;
   const int64_t rows = n * batch * heads;
-  if (quant == PKV_QUANT_Q4K && rows * (a.padded / 256) * 2 <= 1024) {
-    // few superblocks: latency-bound, one workgroup each
-    const int nsb = a.padded / 256;
-    hipLaunchKernelGGL(q4k_append_small_kernel, dim3((unsigned)(2 * rows * nsb)), dim3(256), 0,
-                       s, a, nsb);
-  } else if (quant == PKV_QUANT_Q4K) {
+  // 16-byte loads: rows of a multiple of 4 elements from aligned tensors
+  const bool wide = (a.head_dim & 3) == 0 && ((reinterpret_cast<uintptr_t>(a.src[0]) |
+                                               reinterpret_cast<uintptr_t>(a.src[1])) & 15) == 0;
+  if (quant == PKV_QUANT_Q4K) {
     // 8 kL lanes per superblock: split each sub-block's fit over more lanes while the
-    // append has too few superblocks to give every SIMD a wave
+    // append has too few superblocks to give every SIMD a wave (a workgroup of 256 lanes
+    // per superblock, the fused decode's quantizer, took 6.8 us for 1 to 64 tokens of the
+    // model's shape and 11.1 for 256 where 4 lanes per sub-block take 6.0 and 6.2)
     const int nsb = a.padded / 256;
     const int64_t units = rows * nsb;
     const int kl = 2 * units <= kQ4kAppendLanes4Max ? 4 : (2 * units <= kQ4kAppendLanes2Max ? 2 : 1);
@@ -292,19 +321,34 @@ static int launch_append_args(int quant, AppendArgs &a, hipStream_t s) {
       hipLaunchKernelGGL(q4k_append_kernel<2>, grid, dim3(256), 0, s, a, units, nsb);
     else
       hipLaunchKernelGGL(q4k_append_kernel<1>, grid, dim3(256), 0, s, a, units, nsb);
-  } else if (quant == PKV_QUANT_Q8_0) {
-    const int nblk = a.padded / 32;
-    const int64_t units = rows * nblk;
-    hipLaunchKernelGGL(q8_0_append_kernel, dim3((unsigned)((2 * units + 255) / 256)), dim3(256),
-                       0, s, a, units, nblk);
   } else {
-    const int64_t elems = rows * a.padded;
-    if (quant == PKV_QUANT_BF16)
-      hipLaunchKernelGGL(half_append_kernel<true>, dim3((unsigned)((2 * elems + 255) / 256)),
-                         dim3(256), 0, s, a, elems);
+    const bool q8 = quant == PKV_QUANT_Q8_0, bf = quant == PKV_QUANT_BF16;
+    const int64_t elems = rows * a.padded, blocks = (2 * (elems / 4) + 255) / 256;
+    const bool fit32 = elems / 2 < (1ll << 31);
+    const uint32_t quads = (uint32_t)(elems / 4);
+    const dim3 grid((unsigned)blocks), t(256);
+    // 8-byte stores: rows at multiples of 4 elements
+    const bool half_quads = (a.padded & 3) == 0 && fit32;
+    if (q8 && !fit32)
+      hipLaunchKernelGGL((q8_0_append_kernel<false, uint64_t>), grid, t, 0, s, a, (uint64_t)elems / 4);
+    else if (q8 && wide)
+      hipLaunchKernelGGL((q8_0_append_kernel<true, uint32_t>), grid, t, 0, s, a, quads);
+    else if (q8)
+      hipLaunchKernelGGL((q8_0_append_kernel<false, uint32_t>), grid, t, 0, s, a, quads);
+    else if (half_quads && bf && wide)
+      hipLaunchKernelGGL((half_append_quads_kernel<true, true>), grid, t, 0, s, a, quads);
+    else if (half_quads && bf)
+      hipLaunchKernelGGL((half_append_quads_kernel<true, false>), grid, t, 0, s, a, quads);
+    else if (half_quads && wide)
+      hipLaunchKernelGGL((half_append_quads_kernel<false, true>), grid, t, 0, s, a, quads);
+    else if (half_quads)
+      hipLaunchKernelGGL((half_append_quads_kernel<false, false>), grid, t, 0, s, a, quads);
+    else if (bf)
+      hipLaunchKernelGGL(half_append_kernel<true>, dim3((unsigned)((2 * elems + 255) / 256)), t, 0,
+                         s, a, elems);
     else
-      hipLaunchKernelGGL(half_append_kernel<false>, dim3((unsigned)((2 * elems + 255) / 256)),
-                         dim3(256), 0, s, a, elems);
+      hipLaunchKernelGGL(half_append_kernel<false>, dim3((unsigned)((2 * elems + 255) / 256)), t, 0,
+                         s, a, elems);
   }
   PKV_HIP(hipGetLastError());
   return PKV_OK;

@@ -100,6 +100,32 @@ def test_bulk_append_bitexact(pk, orc, quant):
     assert np.array_equal(host(gk), ok) and np.array_equal(host(gv), ov)
 
 
+@pytest.mark.parametrize("quant,D", [(Q4K, 256), (Q4K, 100), (Q8_0, 256), (Q8_0, 100), (Q8_0, 33), (F16, 256),
+                                     (F16, 36), (F16, 6), (BF16, 64), (BF16, 7)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_append_width_bitexact(pk, orc, quant, D, shift):
+    """Appends of four elements a lane: head_dims that are and are not multiples of 4, K and V
+    that start 0 and 4 bytes past a 16-byte boundary, batches, a few rows and many."""
+    say(f"append width quant={quant} D={D} shift={shift}")
+    rng = np.random.default_rng(500 + quant + D)
+    B, H, cap = 2, 3, 120
+    g = pk.PreallocatedQuantizedKvCache(B, H, cap, D, pk.KvCacheQuantization(quant))
+    c = orc.Cache(quant, B, H, D, cap)
+    for n in (1, 2, 17, 100):
+        k = special_rows(rng, B * H * n, D).reshape(B, H, n, D)
+        v = special_rows(rng, B * H * n, D).reshape(B, H, n, D)[:, :, ::-1].copy()
+        t = []
+        for x in (k, v):
+            big = torch.empty(x.size + 4, device="cuda")
+            t.append(big[shift:shift + x.size].copy_(dev(x).reshape(-1)).reshape(x.shape))
+        assert t[0].data_ptr() % 16 == 4 * shift
+        g.append_quantized(t[0], t[1])
+        assert c.append(k, v) == 0
+    gk, gv = g.raw_bytes()
+    ok, ov = c.valid_bytes()
+    assert np.array_equal(host(gk), ok) and np.array_equal(host(gv), ov)
+
+
 @pytest.mark.parametrize("D,n", [(256, 300), (320, 150), (256, 1500), (320, 700), (256, 2100),
                                  (320, 1100)])
 def test_q4k_append_lane_splits_bitexact(pk, orc, D, n):
