@@ -35,6 +35,7 @@ SOURCES = {
     "pkv_prefill_q8.hip": [],
     "pkv_q8_decode.hip": [],
     "pkv_half_decode.hip": [],
+    "pkv_prefill_half.hip": [],
     "pkv_util.hip": [],
     "pkv_deltanet.hip": [],
     "pkv_oproj.hip": [],

@@ -35,9 +35,11 @@ int launch_append_attend_batched_half(int quant, const SeqDesc *seqs, int n, con
                                       const float *v, const float *q, int num_heads,
                                       int num_kv_heads, int head_dim, float scale, float *out,
                                       Workspace &ws, hipStream_t s);
-// Prefill chunk (l > 1) over Q4K rows of the Qwen3-Next shape (pkv_prefill_mfma.hip).
+// Prefill chunk (l > 1) of the Qwen3-Next shape: Q4K, Q8_0, and F16 / BF16 rows
+// (pkv_prefill_mfma.hip, pkv_prefill_q8.hip, pkv_prefill_half.hip).
 int launch_prefill_mfma(const AttnArgs &a, Workspace &ws, hipStream_t s);
 int launch_prefill_q8_mfma(const AttnArgs &a, Workspace &ws, hipStream_t s);
+int launch_prefill_half(const AttnArgs &a, Workspace &ws, hipStream_t s);
 
 namespace {
 
@@ -252,6 +254,8 @@ int launch_attend(const AttnArgs &a, Workspace &ws, hipStream_t s) {
   rc = launch_prefill_mfma(a, ws, s);
   if (rc != PKV_ERR_UNSUPPORTED) return rc;
   rc = launch_prefill_q8_mfma(a, ws, s);
+  if (rc != PKV_ERR_UNSUPPORTED) return rc;
+  rc = launch_prefill_half(a, ws, s);
   if (rc != PKV_ERR_UNSUPPORTED) return rc;
   return launch_attend_generic(a, ws, s);
 }

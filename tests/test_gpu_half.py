@@ -85,6 +85,26 @@ def test_half_decode_batched(pk, orc, quant):
     assert_attn_close(out, np.stack(refs))
 
 
+@pytest.mark.parametrize("quant", QUANTS)
+@pytest.mark.parametrize("B,S,L,causal", [(1, 0, 2, True), (1, 0, 16, True), (1, 0, 17, True), (1, 31, 33, True),
+                                          (2, 500, 37, True), (1, 700, 3, False), (1, 9000, 5, True),
+                                          (1, 0, 1000, True), (1, 0, 2048, False)])
+def test_half_prefill(pk, orc, B, S, L, causal, quant):
+    """Chunks at tile and block edges, unsplit and with few and many key splits."""
+    say(f"half prefill quant={quant} B={B} S={S} L={L} causal={causal}")
+    rng = np.random.default_rng(S + L)
+    g = pk.PreallocatedQuantizedKvCache(B, 2, S + L, 256, pk.KvCacheQuantization(quant))
+    c = orc.Cache(quant, B, 2, 256, S + L)
+    k, v, q = normal(rng, B, 2, S + L, 256), normal(rng, B, 2, S + L, 256), normal(rng, B, L, 16, 256)
+    k[..., 7] *= 20.0
+    v[..., 9] *= 20.0
+    q[:, :, 3] *= 1e-3
+    g.append_quantized(dev(k), dev(v))
+    assert c.append(k, v) == 0
+    out = g.attend(dev(q), 1 / 16, S, causal)
+    assert_attn_close(out.cpu().numpy(), c.attend(q, 1 / 16, S, causal, mode="f64"))
+
+
 def both(pk, quant, k, v, q, q_offset, causal):
     """(outputs of the aligned rows, outputs of the general kernel: the same rows moved by 8 bytes)."""
     S = k.shape[2]
@@ -106,11 +126,13 @@ def both(pk, quant, k, v, q, q_offset, causal):
 
 @pytest.mark.parametrize("quant", QUANTS)
 @pytest.mark.parametrize("what", ["k_inf", "k_nan", "v_inf", "v_nan", "q_inf", "q_big", "last_v_inf"])
-def test_half_decode_nonfinite(pk, quant, what):
-    say(f"half decode non-finite quant={quant} {what}")
+@pytest.mark.parametrize("l", [1, 20])
+def test_half_nonfinite(pk, quant, what, l):
+    """Also of a key that the causal limit hides from most of a chunk's queries."""
+    say(f"half non-finite quant={quant} {what} l={l}")
     rng = np.random.default_rng(3)
     S = 333
-    k, v, q = normal(rng, 1, 2, S, 256), normal(rng, 1, 2, S, 256), normal(rng, 1, 1, 16, 256)
+    k, v, q = normal(rng, 1, 2, S, 256), normal(rng, 1, 2, S, 256), normal(rng, 1, l, 16, 256)
     if what == "k_inf":
         k[0, 0, 100, 5], k[0, 1, 200, 6] = np.inf, -np.inf
     elif what == "k_nan":
@@ -125,7 +147,25 @@ def test_half_decode_nonfinite(pk, quant, what):
         q[0, 0, 3] *= 1e37
     else:
         v[0, 0, S - 1, 1] = np.inf
-    a, b = both(pk, quant, k, v, q, S - 1, True)
+    a, b = both(pk, quant, k, v, q, S - l, True)
     assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
     # finite values: both are within the attention tolerance of the true ones
     np.testing.assert_allclose(a, b, atol=2e-3, rtol=1e-3)
+
+
+@pytest.mark.parametrize("quant", QUANTS)
+@pytest.mark.parametrize("scale", [0.0, -0.1, 1e-3, 4.0])
+@pytest.mark.parametrize("l", [1, 18])
+def test_half_scales(pk, orc, quant, scale, l):
+    """Scales that no model has: none, a negative one (the general kernel), scores that all
+    but clamp."""
+    say(f"half scale quant={quant} scale={scale} l={l}")
+    rng = np.random.default_rng(11)
+    S = 70
+    g = pk.PreallocatedQuantizedKvCache(1, 2, S, 256, pk.KvCacheQuantization(quant))
+    c = orc.Cache(quant, 1, 2, 256, S)
+    k, v, q = normal(rng, 1, 2, S, 256), normal(rng, 1, 2, S, 256), normal(rng, 1, l, 16, 256)
+    g.append_quantized(dev(k), dev(v))
+    assert c.append(k, v) == 0
+    out = g.attend(dev(q), scale, S - l).cpu().numpy()
+    np.testing.assert_allclose(out, c.attend(q, scale, S - l, True, mode="f64"), atol=2e-3, rtol=1e-3)
