@@ -262,7 +262,9 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(CombineArgsT<kRows>
 // taking entries 4 g .. + 3 of partials ps, ps + 4, ... The form above has 32 slices per 32
 // entries, most of them without a partial then. Step of 4 layers, 16 sequences of 1k to 64k
 // keys: 164.1 -> 162.2 us; 24 paged ones of 0.3k to 12k keys 128.1 -> 124.9 us.
-constexpr int kCombRowMax = 64;
+// Below 8 rows its 16 workgroups per row leave the chip idle: 2 rows of 2000 Q8_0 keys over 12
+// layers 123.4 us, 104.5 in the form above.
+constexpr int kCombRowMax = 64, kCombRows = 8;
 template <int kRows>
 __global__ __launch_bounds__(256) void decode_combine_rows_kernel(CombineArgsT<kRows> c) {
   __shared__ __attribute__((aligned(16))) float acc_s[4][kPartRow];
@@ -572,7 +574,7 @@ static inline int launch_combine(const CombineArgs &c, int n, hipStream_t s) {
   } else {
     int most = 0;
     for (int i = 0; i < n; ++i) most = c.wg1[i] - c.wg0[i] > most ? c.wg1[i] - c.wg0[i] : most;
-    if (most <= kCombRowMax)
+    if (n >= kCombRows && most <= kCombRowMax)
       hipLaunchKernelGGL(decode_combine_rows_kernel<kMaxSegs>, dim3(16, (unsigned)n), dim3(256), 0,
                          s, c);
     else
