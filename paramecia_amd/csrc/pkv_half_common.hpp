@@ -66,12 +66,6 @@ __device__ __forceinline__ T row_load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
   else
     return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
 }
-// LDS written before is visible to the workgroup after; loads from memory stay in flight.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 inline bool half_shape(int quant, int num_heads, int num_kv_heads, int head_dim) {
   return (quant == PKV_QUANT_F16 || quant == PKV_QUANT_BF16) && head_dim == 256 &&

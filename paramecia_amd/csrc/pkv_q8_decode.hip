@@ -21,6 +21,7 @@
 // Fused append: workgroups 0 .. 4 * segments - 1 first quantize one new row each
 // (BlockQ8_0::from_float, bit-exact) and publish it dequantized for the combine.
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "pkv_decode_split.hpp"
@@ -348,8 +349,12 @@ __device__ __forceinline__ void q8_v_codes_dec(const uint32_t (*rows)[kQ8RowWord
 // the decode workgroups need first (segment 0's rows and key count, q, the partial
 // buffers, the row stride, kpw, sl2): the build preloads them into SGPRs, so the first
 // loads of a one-segment launch wait for no kernel-argument fetch.
-template <bool kOne, bool kFused>
-__global__ __launch_bounds__(kQ8mThreads) void q8_decode_mfma_kernel(
+// kMany: more than one block per workgroup. The next block's rows are loaded while this one is
+// worked on (the barriers wait for LDS only), in at most 128 registers so that two
+// workgroups still share a CU: 32768 keys 19.75 to 18.46 us, attend alone. The
+// one-block form without either is 1% faster (4096 keys, 12 layers 104.1 against 105.2 us).
+template <bool kOne, bool kFused, bool kMany>
+__global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_kernel(
     const uint8_t *k_0, const uint8_t *v_0, const float *q, float *part, float2 *mlb, int rs_t,
     int kpw, int seq_k0, float sl2, Q8Args a) {
   __shared__ Q8mSmem sm;
@@ -454,14 +459,17 @@ __global__ __launch_bounds__(kQ8mThreads) void q8_decode_mfma_kernel(
   for (int x = 0; x < 2; ++x) acc[x] = f4{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.0f;  // head n % 8 (the same in lanes n, n ^ 8 and every g)
 
+  const auto sync = [] {
+    if constexpr (kMany) lds_barrier();
+    else __syncthreads();
+  };
   for (int64_t c0 = k0; c0 < k1; c0 += kBlk) {
     const int nk = (int)(k1 - c0 < kBlk ? k1 - c0 : kBlk);
-    if (c0 != k0) {
-      __syncthreads();  // the previous block's readers are done
-      load_block(c0, nk);
-    }
+    if (kMany && c0 != k0) lds_barrier();  // the previous block's readers are done
     store_block(nk);
-    __syncthreads();
+    if (kMany && c0 + kBlk < k1)
+      load_block(c0 + kBlk, (int)(k1 - c0 - kBlk < kBlk ? k1 - c0 - kBlk : kBlk));
+    sync();
     // ---- QK of tile tw over blocks j = 2 qd, 2 qd + 1, A fragments in registers (lane
     // (r, g): key q8_key(r, tw), elements 32 j + 8 g .. + 7)
     f4 cq[2];
@@ -504,7 +512,7 @@ __global__ __launch_bounds__(kQ8mThreads) void q8_decode_mfma_kernel(
       }
       sm.sp[wv][lane] = part;
     }
-    __syncthreads();  // every wave's part of the scores is in LDS
+    sync();  // every wave's part of the scores is in LDS
 
     // ---- the scores: sc[4 t + i] of key 8 g + 4 t + i for column n, summed over the
     // waves' blocks in block order (blocks 0-1, 2-3, 4-5, 6-7)
@@ -637,27 +645,33 @@ static int launch_q8_segments(const DecodeSegIn *in, int n, const float *q, cons
   }
   d.dseg = nullptr;
   d.wps = 0;
-  // The MFMA kernel for caches up to 32768 keys in the standard row layout (both heads'
-  // 272-byte rows adjacent, 16-byte aligned): 32-key blocks, one to four per workgroup
-  // (up to 256 workgroups per segment). Otherwise the VALU kernel: one chunk per
-  // workgroup while that keeps <= 512 partials per segment (16-key chunks up to 8192
-  // keys, 32-key chunks beyond), more chunks per workgroup for longer caches.
-  bool mfma = longest <= 32768 && rs_h == kQ8Row && rs_t % 16 == 0 && rs_t < (1 << 24) &&
+  // The MFMA kernel for caches in the standard row layout (both heads' 272-byte rows
+  // adjacent, 16-byte aligned): 32-key blocks, up to 256 workgroups per KV head and segment
+  // (attend of 40000 / 65536 / 131072 keys: VALU kernel 35.8 / 45.9 / 81.5 us, MFMA 21.5 /
+  // 29.3 / 50.4). Otherwise the VALU kernel: one chunk per workgroup while that keeps <= 512
+  // partials per segment (16-key chunks up to 8192 keys, 32-key chunks beyond), more chunks
+  // per workgroup for longer caches.
+  bool mfma = rs_h == kQ8Row && rs_t % 16 == 0 && rs_t < (1 << 24) &&
               q8_mfma_enabled();
   for (int i = 0; i < n && mfma; ++i)
     mfma = (reinterpret_cast<uintptr_t>(in[i].k) & 15) == 0 &&
            (reinterpret_cast<uintptr_t>(in[i].v) & 15) == 0;
-  int64_t kpw;
-  int chunk;
+  int64_t kpw = (longest + 511) / 512;
+  int chunk = kpw <= 16 ? 16 : kQ8Chunk;
+  kpw = (kpw + chunk - 1) / chunk * chunk;
+  if (kpw < chunk) kpw = chunk;
   if (mfma) {
+    // a no-alloc call over a long cache is accepted when the VALU form's partials fit
+    if (ws.fixed && longest > 32768) {
+      size_t slots = 0;
+      for (int i = 0; i < n; ++i)
+        slots += d.seg[i].seq_k > 0 ? (size_t)((d.seg[i].seq_k + kpw - 1) / kpw) : 1;
+      if (const int rc = ws.reserve((slots * 16 * (kPartRow + 2) + (size_t)n * 4 * 256) * sizeof(float)))
+        return rc;
+    }
     chunk = kBlk;
     kpw = kBlk * ((longest + 256 * kBlk - 1) / (256 * kBlk));
     if (kpw < kBlk) kpw = kBlk;
-  } else {
-    kpw = (longest + 511) / 512;
-    chunk = kpw <= 16 ? 16 : kQ8Chunk;
-    kpw = (kpw + chunk - 1) / chunk * chunk;
-    if (kpw < chunk) kpw = chunk;
   }
   CombineArgs c;
   int wg = 0;
@@ -692,10 +706,15 @@ static int launch_q8_segments(const DecodeSegIn *in, int n, const float *q, cons
       hipLaunchKernelGGL(kern, grid, block, 0, s, d.seg[0].k, d.seg[0].v, q, d.part, d.ml,
                          (int)rs_t, d.kpw, (int)d.seg[0].seq_k, d.sl2, d);
     };
-    if (n == 1 && fused) go(q8_decode_mfma_kernel<true, true>);
-    else if (n == 1) go(q8_decode_mfma_kernel<true, false>);
-    else if (fused) go(q8_decode_mfma_kernel<false, true>);
-    else go(q8_decode_mfma_kernel<false, false>);
+    auto pick = [&](auto many) {
+      constexpr bool kMany = decltype(many)::value;
+      if (n == 1 && fused) go(q8_decode_mfma_kernel<true, true, kMany>);
+      else if (n == 1) go(q8_decode_mfma_kernel<true, false, kMany>);
+      else if (fused) go(q8_decode_mfma_kernel<false, true, kMany>);
+      else go(q8_decode_mfma_kernel<false, false, kMany>);
+    };
+    if (kpw > kBlk) pick(std::true_type{});
+    else pick(std::false_type{});
   } else if (chunk == 16) {
     hipLaunchKernelGGL(q8_decode_kernel<16>, dim3((unsigned)wg), dim3(kQ8Threads), 0, s, d);
   } else {

@@ -251,9 +251,8 @@ def run_decode_q8(pk, orc, S, B=1, fused=True, seed=0, chans=None):
     return np.abs(got - ref).max()
 
 
-# The MFMA kernel takes caches up to 32768 keys (one 32-key block per workgroup up to
-# 8192, two up to 16384, ...: 8223 and 16385 end in a partial block of a workgroup's last
-# pass); 32769 and 40000 take the VALU kernel's 32-key chunks.
+# The MFMA kernel takes one 32-key block per workgroup up to 8192 keys, two up to 16384, ...
+# (five from 32769): 8223 and 16385 end in a partial block of a workgroup's last pass.
 @pytest.mark.parametrize("S", [0, 1, 15, 16, 17, 31, 32, 33, 511, 512, 513, 4096, 8192, 8193,
                                8223, 16385, 20000, 32768, 32769, 40000])
 def test_q8_decode_fused(pk, orc, S):
