@@ -272,7 +272,7 @@ __global__ __launch_bounds__(kQ8Threads) void q8_decode_kernel(Q8Args a) {
   if (kk == 0 && dh == 0) a.ml[(int64_t)wg * 16 + 8 * half + hh] = float2{m_run, l_run};
 }
 
-// ---- MFMA decode over 32-key blocks (caches up to 32k keys per segment)
+// ---- MFMA decode over 32-key blocks
 //
 // A workgroup of 8 waves owns a key range of one segment (kpw keys, a multiple of 32) and
 // one KV head: decode workgroup w (after the quantizing ones) serves partial slot w / 2
@@ -281,15 +281,25 @@ __global__ __launch_bounds__(kQ8Threads) void q8_decode_kernel(Q8Args a) {
 // blocks j = 2 (w % 4), + 1 (int8 codes, exact in fp16) and the PV B fragments of block
 // j = w (its codes, exact in fp16: two 16-column tiles, q8_v_codes_dec). Its QK MFMAs (q
 // as B: columns 0-7 the fp16 hi parts of the group's 8 heads, 8-15 the lo remainders,
-// converted once per workgroup) are scaled by d_j * scale * log2(e) of their keys in
-// f32, and the waves' parts are summed through LDS; the hi and lo columns are summed
-// across lanes n and n ^ 8. The softmax weights times the V d_j of their keys enter PV
-// as A rows 0-7 (fp16 hi) and 8-15 (lo remainder): one MFMA per tile, rows h and h + 8
-// summed at the end. The partial goes out in tile order, as the other decode kernels
-// write it, for decode_combine_kernel.
+// converted once per workgroup) are summed over the two columns of a head, scaled by d_j *
+// scale * log2(e) of their keys in f32, and the waves' parts are summed through LDS. The
+// softmax weights times the V d_j of their keys enter PV as A rows 0-7 (fp16 hi) and 8-15
+// (lo remainder): one MFMA per tile, rows h and h + 8 summed at the end. The partial goes
+// out in tile order, as the other decode kernels write it, for decode_combine_kernel.
+//
+// Both pairs are split at a power of two of their own, undone in f32: 32 q values of a head at
+// their largest, the weights at the largest d_j of the wave's keys so far. A value's hi + lo
+// is then off by 2^-23 of it, or 2^-40 of that largest one. Split as they are, a weight was
+// off by 2^-25 however small V is and |q| >= 65520 became infinite. Relative error against 64
+// bits, N(0, 1) rows: 4096 keys 3.7e-6 (V times 1e-3: 3.7e-3), now 1.7e-7 (1.7e-7); 131072
+// keys 7.2e-6 (7.3e-3), now 2.5e-7 (2.4e-7), the f32 products of the VALU kernel 3.7e-7.
+// Step, us: 4096 keys 7.7 to 7.8, 32768 19.1 to 19.7, 131072 52.5 to 54.1 (VALU 86). As three
+// bf16 parts (exact) in two MFMAs each: 8.0, 20.7, 60.1.
 constexpr int kQ8mThreads = 512;
+constexpr int kVeMin = -24, kVeMax = 15;  // exponents of fp16 values
 struct Q8mSmem {
   h8 qf[8][64];                      // QK B operands: [block j][lane]
+  float qs[8][8];                    // [block j][head]: the power of two to undo
   uint32_t raw[2][32][kQ8RowWords];  // [K / V][key][row]
   float kd[8][32];                   // [block j][key]: K's d_j * sl2 (written when staged)
   float vd[8][32];                   // [block j][key]: V's d_j (written when staged)
@@ -438,14 +448,28 @@ __global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_ker
     const float4 q0 = *reinterpret_cast<const float4 *>(qrow);  // threads >= 256 load again
     const float4 q1 = *reinterpret_cast<const float4 *>(qrow + 4);
     if (k0 < k1) load_block(k0, (int)(k1 - k0 < kBlk ? k1 - k0 : kBlk));
-    if (tid < 256) {
-      const float v8[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+    if (tid < 256) {  // lanes l, l ^ 8 and l ^ 16 hold a head's 32 elements of block j
+      float v8[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+      float mx = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) mx = fmaxf(mx, fabsf(v8[k]));
+      mx = xmax16(fmaxf(mx, ror8(mx)));
+      int e = (int)(f2u(mx) >> 23) - 127;
+      e = e < -100 ? -100 : e > 127 ? 127 : e;
+      const float f = __builtin_ldexpf(1.0f, 14 - e);
+      if (gq == 0) sm.qs[j][hq] = __builtin_ldexpf(1.0f, e - 14);
       h8 fh, fl;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        const _Float16 hi = (_Float16)v8[k];
+        const float x = v8[k] * f;
+        const _Float16 hi = (_Float16)x;
         fh[k] = hi;
-        fl[k] = (_Float16)(v8[k] - (float)hi);
+        fl[k] = (_Float16)(x - (float)hi);
+      }
+      if (__any(mx == INFINITY)) {  // an infinity is its hi part alone (inf - inf is NaN)
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (fabsf(v8[k]) == INFINITY) fl[k] = (_Float16)0.0f;
       }
       sm.qf[j][16 * gq + hq] = fh;
       sm.qf[j][16 * gq + 8 + hq] = fl;
@@ -458,6 +482,7 @@ __global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_ker
 #pragma unroll
   for (int x = 0; x < 2; ++x) acc[x] = f4{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.0f;  // head n % 8 (the same in lanes n, n ^ 8 and every g)
+  int ve = kVeMin;  // the weights' d_j enter times 2^(14 - ve), ve the exponent of the largest
 
   const auto sync = [] {
     if constexpr (kMany) lds_barrier();
@@ -499,16 +524,36 @@ __global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_ker
     q8_v_codes_dec(sm.raw[1], wv, lane, wb);
     const float4 vd0 = *reinterpret_cast<const float4 *>(&sm.vd[wv][8 * g]);
     const float4 vd1 = *reinterpret_cast<const float4 *>(&sm.vd[wv][8 * g + 4]);
-    // this wave's part of its tile's scores, scaled by its keys' d_j, to LDS
+    // the largest d_j (an infinite or NaN one left out) lifts ve
+    const float dv[8] = {vd0.x, vd0.y, vd0.z, vd0.w, vd1.x, vd1.y, vd1.z, vd1.w};
+    float dmax = fabsf(dv[0]);
+#pragma unroll
+    for (int k = 1; k < 8; ++k) dmax = fmaxf(dmax, fabsf(dv[k]));
+    dmax = xmax32(xmax16(dmax));
+    const int de = (__builtin_amdgcn_readfirstlane((int)f2u(dmax)) >> 23) - 127;
+    const bool vinf = de > kVeMax;
+    const int ve_new = de > kVeMax ? kVeMax : de > ve ? de : ve;
+    if (ve_new > ve) {
+      const float down = __builtin_ldexpf(1.0f, ve - ve_new);
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[x][i] *= down;
+      ve = ve_new;
+    }
+    const float vf = __builtin_ldexpf(1.0f, 14 - ve);
+    // this wave's part of its tile's scores, the columns of a head (lanes n and n ^ 8) added
+    // and scaled by its keys' d_j, to LDS
     {
       float4 part = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
         const float4 dk = *reinterpret_cast<const float4 *>(&sm.kd[2 * qd + jj][8 * g + 4 * tw]);
-        part.x = fmaf(dk.x, cq[jj][0], part.x);
-        part.y = fmaf(dk.y, cq[jj][1], part.y);
-        part.z = fmaf(dk.z, cq[jj][2], part.z);
-        part.w = fmaf(dk.w, cq[jj][3], part.w);
+        const float back = sm.qs[2 * qd + jj][n & 7];
+        part.x = fmaf(dk.x, (cq[jj][0] + ror8(cq[jj][0])) * back, part.x);
+        part.y = fmaf(dk.y, (cq[jj][1] + ror8(cq[jj][1])) * back, part.y);
+        part.z = fmaf(dk.z, (cq[jj][2] + ror8(cq[jj][2])) * back, part.z);
+        part.w = fmaf(dk.w, (cq[jj][3] + ror8(cq[jj][3])) * back, part.w);
       }
       sm.sp[wv][lane] = part;
     }
@@ -537,11 +582,12 @@ __global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_ker
       sc[4 * t + 2] = tot.z;
       sc[4 * t + 3] = tot.w;
     }
-    // hi + lo columns (lanes n and n ^ 8), clamp, mask the keys past the range
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      const float s = sc[k] + ror8(sc[k]);
-      sc[k] = 8 * g + k < nk ? fminf(fmaxf(s, -kSplitClampL2), kSplitClampL2) : -INFINITY;
+    for (int k = 0; k < 8; ++k) sc[k] = fminf(fmaxf(sc[k], -kSplitClampL2), kSplitClampL2);
+    if (nk < kBlk) {  // keys past the range
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (8 * g + k >= nk) sc[k] = -INFINITY;
     }
     // ---- online softmax of head n % 8 over the block (lanes n, n + 16, n + 32, n + 48)
     float bm = sc[0];
@@ -552,9 +598,7 @@ __global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_ker
     // some head's max rose after the first block: rescale its sums (rows by head; on the
     // first block they are still 0)
     if (c0 != k0 && __any(m_new != m_run)) {
-      const float alpha = (m_new == m_run) ? 1.0f
-                          : (m_run == -INFINITY) ? 0.0f
-                                                 : __builtin_amdgcn_exp2f(m_run - m_new);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
       l_run *= alpha;
       // row 4 g + i is head (4 g + i) % 8, whose alpha lane (4 g + i) % 8 holds
       const auto lane_alpha = [&](int k) {
@@ -575,20 +619,24 @@ __global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_ker
     m_run = m_new;
     float p[8];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      p[k] = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(sc[k] - m_run);
+    for (int k = 0; k < 8; ++k) {  // (m_run is finite: a block holds a key)
+      p[k] = __builtin_amdgcn_exp2f(sc[k] - m_run);
       l_run += p[k];
     }
     // A rows: n < 8 the fp16 hi parts of head n's weights times d_j of their keys, n >= 8
     // the lo remainders
-    const float dv[8] = {vd0.x, vd0.y, vd0.z, vd0.w, vd1.x, vd1.y, vd1.z, vd1.w};
+    const uint32_t lo_mask = n < 8 ? 0u : 0xFFFFFFFFu;
     uint32_t wa[4];
 #pragma unroll
     for (int k2 = 0; k2 < 4; ++k2) {
-      const float p0 = p[2 * k2] * dv[2 * k2], p1 = p[2 * k2 + 1] * dv[2 * k2 + 1];
-      const uint32_t hw = as_u(h2{(_Float16)p0, (_Float16)p1});
-      const uint32_t lw = fp16_sub2(p0, p1, hw);
-      wa[k2] = n < 8 ? hw : lw;
+      const float p0 = p[2 * k2] * (dv[2 * k2] * vf), p1 = p[2 * k2 + 1] * (dv[2 * k2 + 1] * vf);
+      // fp16(p - c): c = 0 for the hi rows, fp16(p) for the lo rows
+      wa[k2] = fp16_sub2(p0, p1, as_u(h2{(_Float16)p0, (_Float16)p1}) & lo_mask);
+    }
+    if (vinf) {  // an infinite weight is its hi part alone
+#pragma unroll
+      for (int k = 0; k < 8; ++k)
+        if (fabsf(dv[k]) == INFINITY && n >= 8) wa[k >> 1] &= (k & 1) ? 0x0000FFFFu : 0xFFFF0000u;
     }
     const h8 A = __builtin_bit_cast(h8, u4{wa[0], wa[1], wa[2], wa[3]});
 #pragma unroll
@@ -602,11 +650,12 @@ __global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_ker
   // stores: the combine launch reads them from another XCD's L2 misses anyway, and the
   // launch's end then has fewer dirty lines to write back.
   float *P = part + (int64_t)slot * 16 * kPartRow;
+  const float vback = __builtin_ldexpf(1.0f, ve - 14);
   float r[2][4];
 #pragma unroll
   for (int x = 0; x < 2; ++x)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) r[x][i] = xsum32(acc[x][i]);
+    for (int i = 0; i < 4; ++i) r[x][i] = xsum32(acc[x][i]) * vback;
   if (g < 2) {
 #pragma unroll
     for (int x = 0; x < 2; ++x) {

@@ -274,6 +274,77 @@ def test_q8_decode_attend_only(pk, orc, S):
     run_decode_q8(pk, orc, S, fused=False, seed=400 + S)
 
 
+@pytest.mark.parametrize("S,what", [(S, w) for S in (4096, 32768, 40000)
+                                    for w in ("v0.1", "v0.01", "v0.001", "q1e5", "sink")] + [(131072, "v0.001")])
+def test_q8_decode_magnitudes(pk, orc, S, what):
+    """Small V, large q and a first key that outweighs the others by e^14 with a V row of almost
+    nothing, so that the output is made of weights near e^-14: as exact as at N(0, 1)."""
+    say(f"Q8_0 decode {what} S={S}")
+    rng = np.random.default_rng(S)
+    k = rng.standard_normal((1, 2, S + 1, 256)).astype(np.float32)
+    v = rng.standard_normal((1, 2, S + 1, 256)).astype(np.float32)
+    q = rng.standard_normal((1, 1, 16, 256)).astype(np.float32)
+    if what[0] == "v":
+        v *= np.float32(what[1:])
+    elif what == "q1e5":  # beyond fp16's range; scores stay near N(0, 1)
+        q *= np.float32(1e5)
+        k *= np.float32(1e-5)
+    else:
+        u = rng.standard_normal((2, 256)).astype(np.float32)
+        q = 0.2 * q + u[np.arange(16) // 8]
+        k[0, :, 0] = u * np.float32(14 * 16 / 256)
+        v[0, :, 0] *= 1e-3
+    g = pk.PreallocatedQuantizedKvCache(1, 2, S + 1, 256, pk.KvCacheQuantization.Q8_0)
+    c = orc.Cache(Q8_0, 1, 2, 256, S + 1)
+    g.append_quantized(dev(k[:, :, :S]), dev(v[:, :, :S]))
+    assert c.append(k, v) == 0
+    out = g.append_attend(dev(k[:, :, S:]), dev(v[:, :, S:]), dev(q), 1 / 16)
+    l2, _ = assert_attn_close(host(out), c.attend(q, 1 / 16, S, True, mode="f64"))
+    say(f"row error {l2:.2e}")
+
+
+def q8_rows(k, d):
+    """Q8_0 rows of codes k [S, 2, 8, 32] with block scales d [S, 2, 8]."""
+    rows = np.zeros(d.shape[:2] + (8, 34), np.uint8)
+    rows[..., :2] = d.astype(np.float16).view(np.uint8).reshape(d.shape + (2,))
+    rows[..., 2:] = k.view(np.uint8).reshape(d.shape + (32,))
+    return rows.reshape(-1)
+
+
+@pytest.mark.parametrize("S", [77, 9000, 33000])
+@pytest.mark.parametrize("what", ["finite", "k_inf", "v_inf", "v_nan", "q_inf"])
+def test_q8_decode_rows_of_any_scale(pk, what, S):
+    """Codes from -128 on and scales over the whole of fp16, infinities and NaN: what the
+    kernel of rows that are not 16-byte aligned (plain f32 products) gives of the same rows."""
+    say(f"Q8_0 decode rows {what} S={S}")
+    rng = np.random.default_rng(S)
+    codes = [rng.integers(-128, 128, (S, 2, 8, 32)).astype(np.int8) for _ in range(2)]
+    dk = np.exp2(rng.uniform(-14, -7, (S, 2, 8)))
+    dv = np.exp2(rng.uniform(-24, 15, (S, 2, 8)))
+    q = rng.standard_normal((1, 1, 16, 256)).astype(np.float32)
+    if what == "k_inf":
+        dk[S // 2, 0, 3] = np.inf
+    elif what in ("v_inf", "v_nan"):
+        dv[S // 3, 1, 2] = np.inf if what == "v_inf" else np.nan
+    elif what == "q_inf":
+        q[0, 0, 3, 8] = np.inf
+    outs = []
+    for shift in (0, 4):
+        bufs = []
+        for code, d in zip(codes, (dk, dv)):
+            t = torch.zeros(S * 544 + 16, dtype=torch.uint8, device="cuda")
+            t[shift:shift + S * 544] = dev(q8_rows(code, d))
+            bufs.append(t)
+        outs.append(host(pk.flash_attn(pk.KvCacheQuantization.Q8_0, dev(q), bufs[0].data_ptr() + shift,
+                                       bufs[1].data_ptr() + shift, (S * 544, 544, 272, 1), 1 / 16, 2, S, S - 1, True)))
+    a, b = outs
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(np.isinf(a), np.isinf(b))
+    ok = np.isfinite(b)
+    scale = np.abs(np.where(ok, b, 0)).max()
+    # f32 sums of S products, twice
+    assert np.abs(np.where(ok, a, 0) - np.where(ok, b, 0)).max() <= 2e-5 * scale
+
+
 def test_q8_decode_batch2_outliers(pk, orc):
     say("Q8_0 decode batch 2, outlier channels")
     from paramecia_amd import workloads as W
