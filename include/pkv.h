@@ -137,11 +137,11 @@ int pkv_flash_attn(int quant, const float *q, const void *k_bytes, const void *v
 /* pkv_flash_attn for callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). It has no counterpart
  * in the reference. Same arguments, kernels and results as pkv_flash_attn, but the
- * split-K partials go to a library-owned static device array of
- * PKV_NOALLOC_SCRATCH_BYTES on the current device (each GPU holds its own copy until the
- * process ends) instead of an allocated workspace: the call allocates nothing, and a
- * call whose work plan needs more scratch returns PKV_ERR_ARG before it enqueues
- * anything. `stream` must belong to the current device. Every call on one GPU shares that
+ * split-K partials go to a library-owned static device array on the current device (36
+ * MiB; each GPU holds its own copy until the process ends) instead of an allocated
+ * workspace: the call allocates nothing, and a call whose work plan needs more scratch
+ * than PKV_NOALLOC_SCRATCH_BYTES (a prefill chunk: for the splits that fill the GPU, 16 at
+ * most) returns PKV_ERR_ARG before it enqueues anything. `stream` must belong to the current device. Every call on one GPU shares that
  * GPU's array: calls that overlap in time on one GPU (other streams, other threads) race. */
 #define PKV_NOALLOC_SCRATCH_BYTES (16u << 20)
 int pkv_flash_attn_noalloc(int quant, const float *q, const void *k_bytes, const void *v_bytes,

@@ -113,7 +113,7 @@ static int norm_quant(int q) { return q == PKV_QUANT_NONE ? PKV_QUANT_F16 : q; }
 // runs on holds its own copy of this array until the process ends. In host code its name
 // only stands for the symbol: kernels get the device address that hipGetSymbolAddress
 // returns for the current device, looked up once per device and kept.
-static __device__ __align__(256) unsigned char scratch[PKV_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[kNoallocBytes];
 constexpr int kMaxDevices = 64;
 static void *g_scratch_ptr[kMaxDevices];
 static std::mutex g_scratch_mu;

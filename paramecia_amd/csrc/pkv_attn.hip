@@ -194,12 +194,10 @@ static int64_t generic_waves(const AttnArgs &a) {
   wpg = (wpg + kWaves - 1) / kWaves * kWaves;
   return wpg < kWaves ? kWaves : wpg;
 }
-static size_t generic_bytes(const AttnArgs &a) {
+size_t generic_plan_bytes(const AttnArgs &a) {
   const int rows = a.batch * a.l * a.num_heads;
   return (size_t)generic_waves(a) * rows * (2 + (size_t)a.head_dim) * sizeof(float);
 }
-
-int generic_plan_fits(const AttnArgs &a, Workspace &ws) { return ws.reserve(generic_bytes(a)); }
 
 int launch_attend_generic(const AttnArgs &a, Workspace &ws, hipStream_t s) {
   const int G = a.num_heads / a.num_kv_heads;
@@ -208,7 +206,7 @@ int launch_attend_generic(const AttnArgs &a, Workspace &ws, hipStream_t s) {
   const int64_t wpg = generic_waves(a);
   const int64_t kpw = (a.seq_k + wpg - 1) / wpg;
   const int rows = a.batch * a.l * a.num_heads;
-  int rc = ws.reserve(generic_bytes(a));
+  int rc = ws.reserve(generic_plan_bytes(a));
   if (rc) return rc;
   Partials P;
   P.m = reinterpret_cast<float *>(ws.ptr);

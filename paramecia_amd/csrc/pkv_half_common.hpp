@@ -6,8 +6,8 @@
 
 namespace pkv {
 
-// The no-alloc entry accepts a call when the general kernel's plan fits its scratch.
-int generic_plan_fits(const AttnArgs &a, Workspace &ws);
+// Scratch of the general kernel's plan: a no-alloc call is accepted when it fits.
+size_t generic_plan_bytes(const AttnArgs &a);
 
 namespace {
 

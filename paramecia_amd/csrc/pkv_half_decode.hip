@@ -462,7 +462,7 @@ int launch_attend_half(const AttnArgs &a, const float *k_new, const float *v_new
       (reinterpret_cast<uintptr_t>(a.q) & 15) != 0)
     return PKV_ERR_UNSUPPORTED;
   if (ws.fixed)
-    if (const int rc = generic_plan_fits(a, ws)) return rc;
+    if (const int rc = ws.reserve(generic_plan_bytes(a))) return rc;
   for (int b0 = 0; b0 < a.batch; b0 += kMaxSegs) {
     const int nb = a.batch - b0 < kMaxSegs ? a.batch - b0 : kMaxSegs;
     DecodeSegIn in[kMaxSegs];

@@ -61,7 +61,12 @@ struct RowStrides {
 // workspace is destroyed (growth is geometric: they add up to less than 4x the last
 // size). The pinned host buffer stages small descriptor tables; an event guards its
 // reuse. A fixed workspace (fixed = true) wraps caller-provided device memory: reserve()
-// never allocates and refuses a need beyond `bytes` (PKV_ERR_ARG); nothing is freed.
+// never allocates and refuses a need beyond `bytes` (PKV_ERR_ARG); nothing is freed. The
+// no-alloc entry's memory is kNoallocBytes long: a call is accepted by what fits
+// PKV_NOALLOC_SCRATCH_BYTES, and the key splits of an accepted prefill chunk may use the rest
+// (a tile of 16 positions at 128 splits takes 33.8 MB).
+constexpr size_t kNoallocBytes = (size_t)36 << 20;
+static_assert(kNoallocBytes >= PKV_NOALLOC_SCRATCH_BYTES, "what is accepted fits");
 struct Workspace {
   void *ptr = nullptr;
   size_t bytes = 0;

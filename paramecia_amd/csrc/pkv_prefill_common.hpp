@@ -180,7 +180,7 @@ static inline size_t prefill_part_bytes(int batch, int nsplit, int l) {
 // (256 workgroups); a few tokens over a long cache take as many as give every CU a
 // workgroup: 5 tokens over 20016 keys ran 32 workgroups at the earlier limit of 16
 // splits, 98.8 us with the merge; at 128 splits 24.5 us.
-static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk, size_t limit) {
+static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk) {
   constexpr double kPfFixed = 2.0;   // q, the first block's latency, the epilogue
   constexpr double kMergeFixed = 1.5, kMergeBytes = 7e6;  // bytes merged in a block's time
   const int base = ntiles * 2 * a.batch;
@@ -196,7 +196,6 @@ static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk, size_t
   double best_t = 1e30;
   for (int ns = 1; ns <= kMaxMergeSplits && ns <= (nblk > 0 ? nblk : 1); ++ns) {
     const size_t bytes = ns > 1 ? prefill_part_bytes(a.batch, ns, a.l) : 0;
-    if (bytes > limit) break;
     const int64_t rounds = ((int64_t)base * ns + kPfTargetWGs - 1) / kPfTargetWGs;
     const double even = rounds * (mean / ns + kPfFixed), longest = b1 / ns + kPfFixed;
     const double t = (even > longest ? even : longest) +
@@ -209,49 +208,14 @@ static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk, size_t
   return best;
 }
 
-// The plan of a prefill chunk over 32-key blocks: position tiles, key splits, the
-// partials' workspace.
-static inline int prefill_plan(const AttnArgs &a, float sl2, Workspace &ws, PrefillArgs &d) {
-  d.q = a.q;
-  d.k = a.k;
-  d.v = a.v;
-  d.rs_b = a.rs.b;
-  d.rs_t = a.rs.t;
-  d.rs_h = a.rs.h;
-  d.seq_k = a.seq_k;
-  d.q_offset = a.q_offset;
-  d.l = a.l;
-  d.causal = a.causal ? 1 : 0;
-  d.sl2 = sl2;
-  d.ntiles = (a.l + kPosPerWG - 1) / kPosPerWG;
-  const int nblk = (int)((a.seq_k + 31) / 32);
-  size_t limit = ~(size_t)0;
-  if (ws.fixed) {
-    // A no-alloc call is accepted when 256 workgroups' worth of splits (16 at most) fit
-    // the scratch, and then takes no more splits than fit.
-    const int base = d.ntiles * 2 * a.batch;
-    int need = (kPfTargetWGs + base - 1) / base;
-    need = need > 16 ? 16 : need;
-    need = need > nblk ? (nblk > 0 ? nblk : 1) : need;
-    if (need > 1) {
-      const int rc = ws.reserve(prefill_part_bytes(a.batch, need, a.l));
-      if (rc) return rc;
-    }
-    limit = ws.bytes;
-  }
-  const int nsplit = prefill_splits(a, d.ntiles, nblk, limit);
-  d.nsplit = nsplit;
-  d.ngroups = 2 * nsplit * a.batch;
-  d.out = a.out;
-  d.part = nullptr;
-  d.ml = nullptr;
-  if (nsplit > 1) {
-    const int rc = ws.reserve(prefill_part_bytes(a.batch, nsplit, a.l));
-    if (rc) return rc;
-    d.part = static_cast<float *>(ws.ptr);
-    d.ml = reinterpret_cast<float2 *>(d.part + (size_t)a.batch * nsplit * 2 * a.l * 8 * 256);
-  }
-  return PKV_OK;
+// Scratch by which a no-alloc call is accepted: the partials of 256 workgroups' worth of splits
+// (16 at most).
+static inline size_t prefill_accept_bytes(const AttnArgs &a, int ntiles, int nblk) {
+  const int base = ntiles * 2 * a.batch;
+  int need = (kPfTargetWGs + base - 1) / base;
+  need = need > 16 ? 16 : need;
+  need = need > nblk ? (nblk > 0 ? nblk : 1) : need;
+  return need > 1 ? prefill_part_bytes(a.batch, need, a.l) : 0;
 }
 
 // The split merge after a prefill kernel that wrote partials (nsplit > 1).
@@ -264,6 +228,74 @@ static inline int prefill_merge(const PrefillArgs &d, int batch, hipStream_t s) 
     hipLaunchKernelGGL(prefill_merge_wide_kernel, dim3((unsigned)(2 * d.l * 8), (unsigned)batch),
                        dim3(256), 0, s, d.part, d.ml, d.nsplit, d.l, d.out);
   PKV_HIP(hipGetLastError());
+  return PKV_OK;
+}
+
+// Plan and run a prefill chunk over 32-key blocks: launch(d, grid) enqueues the attention
+// kernel, the merge follows. accept_bytes: scratch that a no-alloc call of this shape has to have
+// besides.
+// A no-alloc call uses the splits of an allocating one, so that the two give the same bits.
+// Where their partials exceed its memory, position tiles go through it a group at a time, each a
+// chunk of its own over the same keys. (Fewer splits that fit took 64 us for 32 tokens over
+// 20000 Q4K keys, in place of 46.6.)
+template <typename Launch>
+static inline int prefill_run(const AttnArgs &a, float sl2, Workspace &ws, hipStream_t s,
+                              size_t accept_bytes, Launch launch) {
+  const int ntiles = (a.l + kPosPerWG - 1) / kPosPerWG, nblk = (int)((a.seq_k + 31) / 32);
+  if (ws.fixed) {
+    const size_t bytes = prefill_accept_bytes(a, ntiles, nblk);
+    if (const int rc = ws.reserve(bytes > accept_bytes ? bytes : accept_bytes)) return rc;
+  }
+  const int nsplit = prefill_splits(a, ntiles, nblk);
+  auto run = [&](const AttnArgs &c) -> int {
+    PrefillArgs d;
+    d.q = c.q;
+    d.k = c.k;
+    d.v = c.v;
+    d.rs_b = c.rs.b;
+    d.rs_t = c.rs.t;
+    d.rs_h = c.rs.h;
+    d.seq_k = c.seq_k;
+    d.q_offset = c.q_offset;
+    d.l = c.l;
+    d.causal = c.causal ? 1 : 0;
+    d.sl2 = sl2;
+    d.ntiles = (c.l + kPosPerWG - 1) / kPosPerWG;
+    d.nsplit = nsplit;
+    d.ngroups = 2 * nsplit * c.batch;
+    d.out = c.out;
+    d.part = nullptr;
+    d.ml = nullptr;
+    if (nsplit > 1) {
+      d.part = static_cast<float *>(ws.ptr);
+      d.ml = reinterpret_cast<float2 *>(d.part + (size_t)c.batch * nsplit * 2 * c.l * 8 * 256);
+    }
+    launch(d, dim3((unsigned)(d.ntiles * d.ngroups)));
+    PKV_HIP(hipGetLastError());
+    return prefill_merge(d, c.batch, s);
+  };
+  const size_t part_bytes = nsplit > 1 ? prefill_part_bytes(a.batch, nsplit, a.l) : 0;
+  if (!ws.fixed) {
+    if (const int rc = ws.reserve(part_bytes)) return rc;
+    return run(a);
+  }
+  if (part_bytes <= kNoallocBytes) return run(a);
+  static_assert((size_t)kMaxMergeSplits * 2 * kPosPerWG * 8 * 258 * sizeof(float) <= kNoallocBytes,
+                "a tile's partials fit");
+  const int step = (int)(kNoallocBytes / prefill_part_bytes(1, nsplit, kPosPerWG)) * kPosPerWG;
+  const int64_t q_row = (int64_t)a.num_heads * a.head_dim;
+  for (int b = 0; b < a.batch; ++b)
+    for (int p0 = 0; p0 < a.l; p0 += step) {
+      AttnArgs c = a;
+      c.batch = 1;
+      c.l = a.l - p0 < step ? a.l - p0 : step;
+      c.k = a.k + b * a.rs.b;
+      c.v = a.v + b * a.rs.b;
+      c.q = a.q + ((int64_t)b * a.l + p0) * q_row;
+      c.out = a.out + ((int64_t)b * a.l + p0) * q_row;
+      c.q_offset = a.q_offset + p0;
+      if (const int rc = run(c)) return rc;
+    }
   return PKV_OK;
 }
 

@@ -354,18 +354,13 @@ int launch_prefill_half(const AttnArgs &a, Workspace &ws, hipStream_t s) {
   if (!half_scale(a.scale) || !half_aligned(a.k, a.v, a.rs.b, a.rs.t, a.rs.h) || !decode_rows_fit(a.seq_k, a.rs.t) ||
       ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.out)) & 15) != 0)
     return PKV_ERR_UNSUPPORTED;
-  if (ws.fixed)
-    if (const int rc = generic_plan_fits(a, ws)) return rc;
-  PrefillArgs d;
-  const int rc = prefill_plan(a, a.scale * kLog2e, ws, d);
-  if (rc) return rc;
-  const dim3 grid((unsigned)(d.ntiles * d.ngroups)), block(kPfThreads);
-  if (a.quant == PKV_QUANT_BF16)
-    hipLaunchKernelGGL(half_prefill_kernel<true>, grid, block, 0, s, d);
-  else
-    hipLaunchKernelGGL(half_prefill_kernel<false>, grid, block, 0, s, d);
-  PKV_HIP(hipGetLastError());
-  return prefill_merge(d, a.batch, s);
+  const bool bf = a.quant == PKV_QUANT_BF16;
+  return prefill_run(a, a.scale * kLog2e, ws, s, generic_plan_bytes(a), [&](const PrefillArgs &d, dim3 grid) {
+    if (bf)
+      hipLaunchKernelGGL(half_prefill_kernel<true>, grid, dim3(kPfThreads), 0, s, d);
+    else
+      hipLaunchKernelGGL(half_prefill_kernel<false>, grid, dim3(kPfThreads), 0, s, d);
+  });
 }
 
 }  // namespace pkv

@@ -523,13 +523,9 @@ int launch_prefill_mfma(const AttnArgs &a, Workspace &ws, hipStream_t s) {
   if (a.rs.t >= (1 << 24) || a.seq_k >= (1 << 24) ||
       (uint64_t)a.seq_k * (uint64_t)a.rs.t >= (1ull << 32))
     return PKV_ERR_UNSUPPORTED;
-  PrefillArgs d;
-  const int rc = prefill_plan(a, a.scale * kLog2e, ws, d);
-  if (rc) return rc;
-  hipLaunchKernelGGL(q4k_prefill_kernel, dim3((unsigned)(d.ntiles * d.ngroups)),
-                     dim3(kPfThreads), 0, s, d);
-  PKV_HIP(hipGetLastError());
-  return prefill_merge(d, a.batch, s);
+  return prefill_run(a, a.scale * kLog2e, ws, s, 0, [&](const PrefillArgs &d, dim3 grid) {
+    hipLaunchKernelGGL(q4k_prefill_kernel, grid, dim3(kPfThreads), 0, s, d);
+  });
 }
 
 }  // namespace pkv

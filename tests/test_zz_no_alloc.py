@@ -88,8 +88,31 @@ def test_noalloc_matches_flash_attn_calls_in_a_row(ready):
     compare(pk, Q.Q4K, 2, 5000, 1, 41)
     say("no-alloc: Q8_0 decode, 4097 keys")
     compare(pk, Q.Q8_0, 1, 4097, 1, 42)
-    say("no-alloc: F16 generic path, 3 queries over 700 keys")
+    say("no-alloc: F16, 3 queries over 700 keys")
     compare(pk, Q.F16, 1, 700, 3, 43)
+
+
+@pytest.mark.parametrize("quant", ["q4k", "q8_0"])
+@pytest.mark.parametrize("B,l,S", [(1, 8, 20000), (1, 16, 20000), (1, 32, 20000), (1, 60, 20000),
+                                   (2, 20, 9000), (1, 50, 2000),
+                                   (1, 2500, 5000), (2, 1503, 3503)])
+def test_noalloc_chunks_match_flash_attn(ready, quant, B, l, S):
+    """Chunks whose plan takes more than 16 splits, or partials beyond the static array (the
+    tokens then go through it in groups): the same bits from both entries."""
+    say(f"no-alloc: {quant} {B} x {l} queries over {S} keys")
+    compare(ready, ready.KvCacheQuantization.from_str(quant), B, S, l, 50 + l)
+
+
+def test_noalloc_accepts_60_refuses_64(ready):
+    """The limit lies where it was: 16 splits of 64 tokens are more than 16 MiB."""
+    pk = ready
+    from paramecia_amd._lib import ERR_ARG
+    c = make_cache(pk, pk.KvCacheQuantization.Q4K, 1, 20000, 45)
+    for l, want in ((60, 0), (64, ERR_ARG)):
+        say(f"no-alloc: {l} tokens")
+        q = torch.randn((1, l, 16, 256), device="cuda")
+        out = torch.empty_like(q)
+        assert call("pkv_flash_attn_noalloc", pk.KvCacheQuantization.Q4K, c, q, l, 20000 - l, True, out) == want
 
 
 def test_noalloc_refuses_plan_beyond_scratch(ready):
