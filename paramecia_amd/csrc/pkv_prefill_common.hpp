@@ -21,6 +21,7 @@ constexpr int kPfTargetWGs = 256;
 constexpr float kPfLazy = 8.0f;
 constexpr int kNarrowSplits = 16;    // splits the narrow merge takes (all loads in flight)
 constexpr int kMaxMergeSplits = 128;  // splits the wide merge takes
+constexpr size_t kPfMaxPartBytes = (size_t)256 << 20;
 
 struct PrefillArgs {
   const float *q;  // [B][l][16][256]
@@ -179,7 +180,8 @@ static inline size_t prefill_part_bytes(int batch, int nsplit, int l) {
 // A chunk that fills the GPU by itself keeps one split; 512 tokens over 16896 keys take 4
 // (256 workgroups); a few tokens over a long cache take as many as give every CU a
 // workgroup: 5 tokens over 20016 keys ran 32 workgroups at the earlier limit of 16
-// splits, 98.8 us with the merge; at 128 splits 24.5 us.
+// splits, 98.8 us with the merge; at 128 splits 24.5 us. The partials take kPfMaxPartBytes
+// at most: beyond lie chunks of many rows that fill the GPU without a split.
 static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk) {
   constexpr double kPfFixed = 2.0;   // q, the first block's latency, the epilogue
   constexpr double kMergeFixed = 1.5, kMergeBytes = 7e6;  // bytes merged in a block's time
@@ -196,6 +198,7 @@ static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk) {
   double best_t = 1e30;
   for (int ns = 1; ns <= kMaxMergeSplits && ns <= (nblk > 0 ? nblk : 1); ++ns) {
     const size_t bytes = ns > 1 ? prefill_part_bytes(a.batch, ns, a.l) : 0;
+    if (bytes > kPfMaxPartBytes) break;
     const int64_t rounds = ((int64_t)base * ns + kPfTargetWGs - 1) / kPfTargetWGs;
     const double even = rounds * (mean / ns + kPfFixed), longest = b1 / ns + kPfFixed;
     const double t = (even > longest ? even : longest) +

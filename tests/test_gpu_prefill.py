@@ -170,3 +170,20 @@ def test_prefill_full_chunk(pk, orc, quant):
     err = np.abs(out - ref)
     say(f"full prefill chunk quant={quant}: max|diff| = {err.max():.3e}")
     assert_attn_close(out, ref)
+
+
+def test_prefill_partials_stay_bounded(pk):
+    """A batch of chunks over long caches, which the GPU could run in 5 key splits (378 MB of
+    partials): the plan's partials stay within 256 MiB, a workspace within 5 / 4 of that."""
+    say("prefill: 16 x 300 tokens over 40300 keys")
+    B, S, L = 16, 40000, 300
+    c = pk.PreallocatedQuantizedKvCache(B, 2, S + L, 256, pk.KvCacheQuantization.Q4K)
+    c.set_len(S + L)
+    q = torch.randn((B, L, 16, 256), device="cuda")
+    out = torch.empty_like(q)
+    del out  # torch keeps the memory for the call's output
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    c.attend(q, 1 / 16, S)
+    torch.cuda.synchronize()
+    assert before - torch.cuda.mem_get_info()[0] <= (256 << 20) * 5 // 4 + (4 << 20)
