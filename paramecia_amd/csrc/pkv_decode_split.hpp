@@ -259,12 +259,14 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(CombineArgsT<kRows>
 }
 // Rows of at most kCombRowMax partials (a serving batch: its 256 workgroups' partials shared
 // out over the rows): one workgroup per (head, row), 4 slices of 64 threads, thread (ps, g)
-// taking entries 4 g .. + 3 of partials ps, ps + 4, ... The form above has 32 slices per 32
-// entries, most of them without a partial then. Step of 4 layers, 16 sequences of 1k to 64k
-// keys: 164.1 -> 162.2 us; 24 paged ones of 0.3k to 12k keys 128.1 -> 124.9 us.
-// Below 8 rows its 16 workgroups per row leave the chip idle: 2 rows of 2000 Q8_0 keys over 12
-// layers 123.4 us, 104.5 in the form above.
-constexpr int kCombRowMax = 64, kCombRows = 8;
+// taking entries 4 g .. + 3 of partials ps, ps + 4, ..., all in flight at once. The form above
+// has 32 slices per 32 entries, most of them without a partial then.
+// Taken from kCombRows rows on. us after a kernel that writes the partials, form above / this
+// one, rows x partials: 6 x 8 2.8 / 3.0, 6 x 32 4.2 / 4.3 (16 workgroups a row leave the chip
+// idle); 8 x 8 3.2 / 3.2, 8 x 32 5.0 / 4.3; 16 x 4 4.4 / 3.2, 16 x 32 7.5 / 6.0; 32 x 8 7.9 /
+// 4.7, 32 x 32 12.9 / 9.5. A second round of loads (33 partials and more) does not pay at few
+// rows: 8 x 40 5.1 / 6.0, 16 x 64 10.0 / 10.4, 32 x 40 13.7 / 12.3.
+constexpr int kCombRowMax = 4 * kCombChunk, kCombRows = 8;
 template <int kRows>
 __global__ __launch_bounds__(256) void decode_combine_rows_kernel(CombineArgsT<kRows> c) {
   __shared__ __attribute__((aligned(16))) float acc_s[4][kPartRow];
@@ -275,17 +277,14 @@ __global__ __launch_bounds__(256) void decode_combine_rows_kernel(CombineArgsT<k
   const float2 *ML = c.ml + (int64_t)wbeg * 16 + h;
   float2 mlv[kCombChunk];
   float4 ov[kCombChunk];
-  auto load_round = [&](int w) {  // past the partials: the first one's, with no weight
 #pragma unroll
-    for (int x = 0; x < kCombChunk; ++x) {
-      const bool ok = w + 4 * x < np;
-      const int64_t i = ok ? w + 4 * x : 0;
-      const float2 t = ML[i * 16];
-      ov[x] = *reinterpret_cast<const float4 *>(P + i * 16 * kPartRow);
-      mlv[x] = ok ? t : float2{-INFINITY, 0.0f};
-    }
-  };
-  load_round(ps);
+  for (int x = 0; x < kCombChunk; ++x) {  // past the partials: the first one's, with no weight
+    const bool ok = ps + 4 * x < np;
+    const int64_t i = ok ? ps + 4 * x : 0;
+    const float2 t = ML[i * 16];
+    ov[x] = *reinterpret_cast<const float4 *>(P + i * 16 * kPartRow);
+    mlv[x] = ok ? t : float2{-INFINITY, 0.0f};
+  }
   const int e = tile_e(tid >> 4, tid & 15);
   const bool has_new = c.dq != nullptr;
   float qk = 0.0f, vnew = 0.0f;
@@ -295,29 +294,17 @@ __global__ __launch_bounds__(256) void decode_combine_rows_kernel(CombineArgsT<k
   }
   float m = -INFINITY, l = 0.0f;
   float4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (int w = ps; w < np; w += 4 * kCombChunk) {
-    if (w != ps) load_round(w);
-    float mc = m;
 #pragma unroll
-    for (int x = 0; x < kCombChunk; ++x) mc = fmaxf(mc, mlv[x].x);
-    if (mc == -INFINITY) continue;
-    const float r = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mc);
-    acc.x *= r;
-    acc.y *= r;
-    acc.z *= r;
-    acc.w *= r;
-    l *= r;
+  for (int x = 0; x < kCombChunk; ++x) m = fmaxf(m, mlv[x].x);
 #pragma unroll
-    for (int x = 0; x < kCombChunk; ++x) {
-      if (mlv[x].x == -INFINITY) continue;
-      const float f = __builtin_amdgcn_exp2f(mlv[x].x - mc);
-      acc.x += f * ov[x].x;
-      acc.y += f * ov[x].y;
-      acc.z += f * ov[x].z;
-      acc.w += f * ov[x].w;
-      l += f * mlv[x].y;
-    }
-    m = mc;
+  for (int x = 0; x < kCombChunk; ++x) {
+    if (mlv[x].x == -INFINITY) continue;
+    const float f = __builtin_amdgcn_exp2f(mlv[x].x - m);
+    acc.x += f * ov[x].x;
+    acc.y += f * ov[x].y;
+    acc.z += f * ov[x].z;
+    acc.w += f * ov[x].w;
+    l += f * mlv[x].y;
   }
   const float d = wave_sum(qk);
   *reinterpret_cast<float4 *>(&acc_s[ps][4 * g]) = acc;

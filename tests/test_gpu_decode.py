@@ -134,14 +134,14 @@ def test_decode_full_size_layer(pk, orc):
     assert_attn_close(out, ref)
 
 
-def run_batched(pk, orc, lens, seed, chans=None):
+def run_batched(pk, orc, lens, seed, chans=None, quant=Q4K):
     """One batched decode step over len(lens) caches of different lengths: each gets a
     new token appended (bit-exact bytes) and its query attends over all its keys."""
     rng = np.random.default_rng(seed)
     caches, oracles = [], []
     for S in lens:
-        g = pk.PreallocatedQuantizedKvCache(1, 2, S + 1, 256, pk.KvCacheQuantization.Q4K)
-        c = orc.Cache(Q4K, 1, 2, 256, S + 1)
+        g = pk.PreallocatedQuantizedKvCache(1, 2, S + 1, 256, pk.KvCacheQuantization(quant))
+        c = orc.Cache(quant, 1, 2, 256, S + 1)
         if S > 0:
             k = rng.standard_normal((1, 2, S, 256)).astype(np.float32)
             v = rng.standard_normal((1, 2, S, 256)).astype(np.float32)
@@ -378,6 +378,15 @@ def test_q8_batched_varlen(pk, orc):
         gk, gv = g.raw_bytes()
         ok, ov = c.valid_bytes()
         assert np.array_equal(host(gk), ok) and np.array_equal(host(gv), ov)
+
+
+@pytest.mark.parametrize("lens", [[1024] * 7 + [5], [1025] + [40] * 7, [1024] * 7, [992, 1, 0, 33] * 8],
+                         ids=["8x32", "8x33", "7x32", "32x31"])
+def test_combine_forms(pk, orc, lens):
+    """A Q8_0 sequence has one partial per 32 keys: rows and partials on either side of where
+    the combine with one workgroup per head and row is taken (8 rows, 32 partials)."""
+    say(f"combine of {len(lens)} rows of up to {max(lens)} keys")
+    run_batched(pk, orc, lens, seed=len(lens), quant=Q8_0)
 
 
 def test_inlaunch_combine_replays_and_mixed_sizes(pk, orc):
