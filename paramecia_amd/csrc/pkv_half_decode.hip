@@ -24,7 +24,7 @@
 // per block and KV head with its merge in LDS (14.4 at 100 keys, 16.0 at 12290: one wave's
 // serial work), 384 and 512 slots (14.4 and 15.1 at 12290: the combine reads more).
 // Precision: q and the weights p enter as sums of 16-bit parts, accumulated in f32: F16 hi
-// and lo (q scaled by a power of two per row, p by 2^7, so that neither part leaves fp16's
+// and lo (q scaled by a power of two per row, p by 2^11, so that neither part leaves fp16's
 // range: 22 bits), BF16 three parts (24 bits). Mean error against 64 bits over 20 to 12000
 // keys with scores of standard deviation 0.01 / 1 / 4: 0.24 to 1.1 times the general
 // kernel's (12000 keys, 1: F16 1.9e-7 of 5.2e-7).
@@ -43,7 +43,6 @@ namespace {
 
 constexpr int kHdWaves = 4, kHdThreads = 64 * kHdWaves;
 constexpr int kHdSlots = 256;  // partial slots of a full launch, two workgroups (KV heads) each
-constexpr float kHdLazy = 8.0f;    // log2 headroom of the running max before a rescale
 
 struct HalfSeg {
   uint8_t *k, *v;  // rows of token 0, KV head 0
@@ -222,10 +221,10 @@ __global__ __launch_bounds__(kHdThreads) void half_decode_kernel(
   for (int j = 0; j < 4; ++j) acc[j] = zero;
   // Scores and the running max stay in q . k units; each exponent is the fma of the score's
   // two summands (rounding a score of tens of log2 units instead cost 2-4 times the error
-  // where a few keys dominate, one fma of the rounded sum 1.3 times). F16's factor 2^7 is a product of its own: in the exponent it would
+  // where a few keys dominate, one fma of the rounded sum 1.3 times). F16's factor 2^11 is a product of its own: in the exponent it would
   // round the small ones of the keys that matter.
   constexpr float kUp = kBf ? 1.0f : kPUp;
-  const float cs = a.sl2, clamp = kClampL2 / cs, lazy = kHdLazy / cs;
+  const float cs = a.sl2, clamp = kClampL2 / cs, lazy = (kBf ? kBf16Lazy : kF16Lazy) / cs;
   float m_run = -INFINITY, nm = INFINITY, lsum = 0.0f;
   bool bad = false;
   for (int b = b0; b < b1; ++b) {

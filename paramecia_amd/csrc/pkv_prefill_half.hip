@@ -203,7 +203,7 @@ __global__ __launch_bounds__(kPfThreads) void half_prefill_kernel(PrefillArgs a)
 #pragma unroll
   for (int T = 0; T < 16; ++T) acc[T] = zero;
   constexpr float kUp = kBf ? 1.0f : kPUp;  // (not in the exponents: it would round them)
-  const float clamp = kClampL2 / cs, lazy = kPfLazy / cs;
+  const float clamp = kClampL2 / cs, lazy = (kBf ? kBf16Lazy : kF16Lazy) / cs;
   float m_run = -INFINITY, nm = INFINITY, lsum = 0.0f;
   bool bad = false;
   const int64_t klim = a.causal ? (int64_t)pw + (n >> 3) + a.q_offset : (int64_t)1 << 62;
