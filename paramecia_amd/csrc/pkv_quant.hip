@@ -101,16 +101,15 @@ __global__ __launch_bounds__(256) void q4k_append_kernel(AppendArgs a, int64_t u
 }
 
 // Four elements of a row per lane: 16-byte loads where kWide (head_dim a multiple of 4, K
-// and V 16-byte aligned), else one by one. U counts lanes: 32 bits but for appends of 2^31
-// lanes and more. A lane's tensor p, row (t, b, h) and elements e .. e + 3; false past the end.
+// and V 16-byte aligned), else one by one. U counts quads: 32 bits but for appends of 2^31
+// quads and more. Quad i's tensor p, row (t, b, h) and elements e .. e + 3; false past the end.
 struct Quad {
   float x[4];
   int p, b, h, e;
   int64_t t;
 };
 template <bool kWide, typename U>
-__device__ __forceinline__ bool load_quad(const AppendArgs &a, U quads_per_tensor, Quad &q) {
-  const U i = (U)blockIdx.x * 256 + threadIdx.x;
+__device__ __forceinline__ bool load_quad(const AppendArgs &a, U quads_per_tensor, U i, Quad &q) {
   if (i >= 2 * quads_per_tensor) return false;
   q.p = i >= quads_per_tensor;
   const U u = q.p ? i - quads_per_tensor : i;
@@ -141,10 +140,11 @@ __device__ __forceinline__ bool load_quad(const AppendArgs &a, U quads_per_tenso
 // wave reads 1 KB and writes 272 bytes in a row. The block's largest |x| is exact in any
 // order (NaN dropped, as f32::max does). One lane per block, with 32 scalar loads and 17
 // 2-byte stores, took 11.0 us for 512 tokens of the model's shape (2.7 MB), this form 3.3 us.
+// With 64-bit counts the lanes go on by the grid's size: a launch holds fewer than 2^32.
 template <bool kWide, typename U>
-__global__ __launch_bounds__(256) void q8_0_append_kernel(AppendArgs a, U quads_per_tensor) {
+__device__ __forceinline__ bool q8_0_append_quad(const AppendArgs &a, U quads_per_tensor, U i) {
   Quad q;
-  if (!load_quad<kWide, U>(a, quads_per_tensor, q)) return;
+  if (!load_quad<kWide, U>(a, quads_per_tensor, i, q)) return false;
   int32_t key = 0;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -167,6 +167,16 @@ __global__ __launch_bounds__(256) void q8_0_append_kernel(AppendArgs a, U quads_
   o[0] = (uint16_t)w;
   o[1] = (uint16_t)(w >> 16);
   if ((q.e & 31) == 0) *reinterpret_cast<uint16_t *>(blk) = f32_to_f16(d);
+  return true;
+}
+template <bool kWide, typename U>
+__global__ __launch_bounds__(256) void q8_0_append_kernel(AppendArgs a, U quads_per_tensor) {
+  U i = (U)blockIdx.x * 256 + threadIdx.x;
+  if constexpr (sizeof(U) == 4) {
+    q8_0_append_quad<kWide, U>(a, quads_per_tensor, i);
+  } else {
+    while (q8_0_append_quad<kWide, U>(a, quads_per_tensor, i)) i += (U)gridDim.x * 256;
+  }
 }
 
 // F16 / BF16 rows: round-to-nearest-even conversion, four elements a lane (4096 tokens of
@@ -176,7 +186,7 @@ template <bool BF, bool kWide>
 __global__ __launch_bounds__(256) void half_append_quads_kernel(AppendArgs a,
                                                                 uint32_t quads_per_tensor) {
   Quad q;
-  if (!load_quad<kWide, uint32_t>(a, quads_per_tensor, q)) return;
+  if (!load_quad<kWide, uint32_t>(a, quads_per_tensor, blockIdx.x * 256 + threadIdx.x, q)) return;
   uint32_t y[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) y[k] = BF ? f32_to_bf16(q.x[k]) : f32_to_f16(q.x[k]);
@@ -330,7 +340,7 @@ static int launch_append_args(int quant, AppendArgs &a, hipStream_t s) {
     // 8-byte stores: rows at multiples of 4 elements
     const bool half_quads = (a.padded & 3) == 0 && fit32;
     if (q8 && !fit32)
-      hipLaunchKernelGGL((q8_0_append_kernel<false, uint64_t>), grid, t, 0, s, a, (uint64_t)elems / 4);
+      hipLaunchKernelGGL((q8_0_append_kernel<false, uint64_t>), dim3(1u << 20), t, 0, s, a, (uint64_t)elems / 4);
     else if (q8 && wide)
       hipLaunchKernelGGL((q8_0_append_kernel<true, uint32_t>), grid, t, 0, s, a, quads);
     else if (q8)

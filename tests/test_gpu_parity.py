@@ -573,3 +573,30 @@ def test_allocating_calls_refused_under_capture(pk):
     assert L.pkv_prefix_free(pre) == 0
     g.resize_batch(2)
     assert g.batch_size == 2
+
+
+def test_q8_append_of_2_33_elements(pk, orc):
+    """One Q8_0 append whose four-element groups number 2^32 and more: the rows at its ends and
+    around the 2^31st and 2^32nd group, and a row of zeros."""
+    if torch.cuda.mem_get_info()[0] < 80 << 30:
+        pytest.skip("needs 80 GB of GPU memory")
+    say("Q8_0 append of 2^33 elements")
+    heads, d = 8, 512
+    n = (1 << 33) // (heads * d) + 3
+    x = torch.zeros((1, heads, n, d), device="cuda")
+    rng = np.random.default_rng(33)
+    at = [0, 1, n // 2 - 2, n // 2 - 1, n // 2, n // 2 + 1, n - 5, n - 4, n - 2, n - 1]
+    rows = rng.standard_normal((1, heads, len(at), d)).astype(np.float32)
+    x[:, :, at] = torch.from_numpy(rows).cuda()
+    c = pk.PreallocatedQuantizedKvCache(1, heads, n, d, pk.KvCacheQuantization.Q8_0)
+    c.append_quantized(x, x)
+    del x
+    want = orc.Cache(3, 1, heads, d, len(at))
+    assert want.append(rows, rows) == 0
+    bytes_ = want.valid_bytes()[0].reshape(len(at), -1)
+    for got in c.raw_bytes():
+        got = got.view(n, -1)
+        assert np.array_equal(got[at].cpu().numpy(), bytes_)
+        assert not got[n // 4].any() and not got[n - 3].any()
+    del got, c
+    torch.cuda.empty_cache()
