@@ -959,7 +959,16 @@ __global__ __launch_bounds__(kThreads) void q4k_decode_kernel(
         // first ones quantize); the in-launch combiners, on other XCDs, read it once the
         // word below has the launch's parity.
         const bool publish = (kOne ? wg == nwg_0 - 1 : wg == sg.wg0) && wsub == 0;
-        if (publish && n < 8) {
+        if (publish && n < 8 && !kOne) {  // read by the next launch: plain stores
+          float *qo = a.q_out + ((int64_t)sg.qi * 16 + 8 * kvu + n) * 256 + 64 * g;
+#pragma unroll
+          for (int st = 0; st < 8; ++st)
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+              *reinterpret_cast<float4 *>(qo + 8 * st + 4 * x) =
+                  float4{v[st][4 * x], v[st][4 * x + 1], v[st][4 * x + 2], v[st][4 * x + 3]};
+        }
+        if (publish && n < 8 && kOne) {
           float *qo = a.q_out + ((int64_t)sg.qi * 16 + 8 * kvu) * 256;
           // (16-byte agent-scope stores: as 64 dword stores per lane they held the
           // workgroup up: 24.9 us per step at 32768 keys, 19.8 now)
