@@ -359,12 +359,17 @@ __device__ __forceinline__ void q8_v_codes_dec(const uint32_t (*rows)[kQ8RowWord
 // the decode workgroups need first (segment 0's rows and key count, q, the partial
 // buffers, the row stride, kpw, sl2): the build preloads them into SGPRs, so the first
 // loads of a one-segment launch wait for no kernel-argument fetch.
-// kMany: more than one block per workgroup. The next block's rows are loaded while this one is
-// worked on (the barriers wait for LDS only), in at most 128 registers so that two
-// workgroups still share a CU: 32768 keys 19.75 to 18.46 us, attend alone. The
-// one-block form without either is 1% faster (4096 keys, 12 layers 104.1 against 105.2 us).
-template <bool kOne, bool kFused, bool kMany>
-__global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_kernel(
+// kForm: kQ8Many, more than one block per workgroup. The next block's rows are loaded while this
+// one is worked on (the barriers wait for LDS only), in at most 128 registers so that two
+// workgroups still share a CU: 32768 keys 19.75 to 18.46 us, attend alone. kQ8Full, one block
+// and two workgroups per CU or more: as straight code, which the compiler puts into 56
+// registers, so that four share a CU. kQ8Few, one block and fewer workgroups: compiled as a
+// loop, with its loads and LDS reads issued earlier in 122 registers. us per step, kQ8Few /
+// kQ8Full: 1 x 4000 keys 7.9 / 8.0 (250 workgroups), 1 x 8192 10.6 / 10.35 (512), 2 x 6000
+// 14.2 / 12.8, 4 x 6686 24.6 / 20.3, 8 x 8192 55.9 / 43.6.
+enum { kQ8Few, kQ8Full, kQ8Many };
+template <bool kOne, bool kFused, int kForm>
+__global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_decode_mfma_kernel(
     const uint8_t *k_0, const uint8_t *v_0, const float *q, float *part, float2 *mlb, int rs_t,
     int kpw, int seq_k0, float sl2, Q8Args a) {
   __shared__ Q8mSmem sm;
@@ -485,14 +490,14 @@ __global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_ker
   int ve = kVeMin;  // the weights' d_j enter times 2^(14 - ve), ve the exponent of the largest
 
   const auto sync = [] {
-    if constexpr (kMany) lds_barrier();
+    if constexpr (kForm == kQ8Many) lds_barrier();
     else __syncthreads();
   };
   for (int64_t c0 = k0; c0 < k1; c0 += kBlk) {
     const int nk = (int)(k1 - c0 < kBlk ? k1 - c0 : kBlk);
-    if (kMany && c0 != k0) lds_barrier();  // the previous block's readers are done
+    if (kForm == kQ8Many && c0 != k0) lds_barrier();  // the previous block's readers are done
     store_block(nk);
-    if (kMany && c0 + kBlk < k1)
+    if (kForm == kQ8Many && c0 + kBlk < k1)
       load_block(c0 + kBlk, (int)(k1 - c0 - kBlk < kBlk ? k1 - c0 - kBlk : kBlk));
     sync();
     // ---- QK of tile tw over blocks j = 2 qd, 2 qd + 1, A fragments in registers (lane
@@ -642,6 +647,7 @@ __global__ __launch_bounds__(kQ8mThreads, kMany ? 4 : 2) void q8_decode_mfma_ker
 #pragma unroll
     for (int x = 0; x < 2; ++x)
       acc[x] = mfma32(A, __builtin_bit_cast(h8, u4{wb[x][0], wb[x][1], wb[x][2], wb[x][3]}), acc[x]);
+    if constexpr (kForm == kQ8Full) break;
   }
 
   // ---- partial: rows h (hi weights) and h + 8 (lo) summed (lanes g and g + 2); element
@@ -755,15 +761,16 @@ static int launch_q8_segments(const DecodeSegIn *in, int n, const float *q, cons
       hipLaunchKernelGGL(kern, grid, block, 0, s, d.seg[0].k, d.seg[0].v, q, d.part, d.ml,
                          (int)rs_t, d.kpw, (int)d.seg[0].seq_k, d.sl2, d);
     };
-    auto pick = [&](auto many) {
-      constexpr bool kMany = decltype(many)::value;
-      if (n == 1 && fused) go(q8_decode_mfma_kernel<true, true, kMany>);
-      else if (n == 1) go(q8_decode_mfma_kernel<true, false, kMany>);
-      else if (fused) go(q8_decode_mfma_kernel<false, true, kMany>);
-      else go(q8_decode_mfma_kernel<false, false, kMany>);
+    auto pick = [&](auto form) {
+      constexpr int kForm = decltype(form)::value;
+      if (n == 1 && fused) go(q8_decode_mfma_kernel<true, true, kForm>);
+      else if (n == 1) go(q8_decode_mfma_kernel<true, false, kForm>);
+      else if (fused) go(q8_decode_mfma_kernel<false, true, kForm>);
+      else go(q8_decode_mfma_kernel<false, false, kForm>);
     };
-    if (kpw > kBlk) pick(std::true_type{});
-    else pick(std::false_type{});
+    if (kpw > kBlk) pick(std::integral_constant<int, kQ8Many>{});
+    else if (2 * wg >= 512) pick(std::integral_constant<int, kQ8Full>{});
+    else pick(std::integral_constant<int, kQ8Few>{});
   } else if (chunk == 16) {
     hipLaunchKernelGGL(q8_decode_kernel<16>, dim3((unsigned)wg), dim3(kQ8Threads), 0, s, d);
   } else {
