@@ -380,6 +380,41 @@ def test_q8_batched_varlen(pk, orc):
         assert np.array_equal(host(gk), ok) and np.array_equal(host(gv), ov)
 
 
+@pytest.mark.parametrize("lens", [[0, 33, 8193, 20000, 40000], [8000, 1, 8192, 31, 4100]],
+                         ids=["pipelined", "full"])
+def test_q8_batched_long(pk, orc, lens):
+    """Several sequences whose workgroups take five blocks each (40000 keys: 160 per workgroup),
+    or one block each of more than 512 workgroups."""
+    say(f"Q8_0 batched decode {lens}")
+    run_batched(pk, orc, lens, seed=len(lens) + lens[0], quant=Q8_0)
+
+
+@pytest.mark.parametrize("B,S,fused", [(2, 9001, False), (3, 3001, True), (2, 9001, True)])
+def test_q8_decode_rows(pk, orc, B, S, fused):
+    say(f"Q8_0 decode B={B} S={S} fused={fused}")
+    run_decode_q8(pk, orc, S, B=B, fused=fused, seed=S + B)
+
+
+def test_q8_decode_without_mfma():
+    """The f32 kernel with an append (both chunk sizes, one and two rows): it is left to batches
+    whose rows are 16 MiB apart and more, so a process of its own turns the MFMA form off."""
+    import os
+    import subprocess
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    here = os.path.dirname(os.path.abspath(__file__))
+    root = os.path.dirname(here)
+    code = ("import sys; sys.path[:0] = %r\n"
+            "import oracle, paramecia_amd, test_gpu_decode as t\n"
+            "for B, S in ((1, 0), (1, 1), (1, 33), (2, 3000), (1, 8193), (1, 40000)):\n"
+            "    t.say(B, S, t.run_decode_q8(paramecia_amd, oracle, S, B=B, seed=S))\n"
+            % [root, os.path.join(root, "oracle"), here])
+    r = subprocess.run([sys.executable, "-c", code], env=dict(os.environ, PKV_Q8_MFMA="0"),
+                       capture_output=True, text=True, timeout=100)
+    say(r.stdout, r.stderr[-2000:])
+    assert r.returncode == 0
+
+
 @pytest.mark.parametrize("lens", [[1024] * 7 + [5], [1025] + [40] * 7, [1024] * 7, [992, 1, 0, 33] * 8],
                          ids=["8x32", "8x33", "7x32", "32x31"])
 def test_combine_forms(pk, orc, lens):

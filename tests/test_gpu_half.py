@@ -66,8 +66,19 @@ def test_half_decode(pk, orc, B, S, quant):
 def test_half_decode_batched(pk, orc, quant):
     """Sequences of 0 to 3000 keys in one call, more of them than a launch takes."""
     say(f"half decode batched quant={quant}")
+    run_half_batched(pk, orc, quant, 3000)
+
+
+@pytest.mark.parametrize("quant", QUANTS)
+def test_half_decode_batched_few_partials(pk, orc, quant):
+    """At most 700 keys, 22 partials: the combine with one workgroup per head and row."""
+    say(f"half decode batched, few partials quant={quant}")
+    run_half_batched(pk, orc, quant, 700)
+
+
+def run_half_batched(pk, orc, quant, most):
     rng = np.random.default_rng(7)
-    lens = [0, 1, 32, 33, 3000, 64] + [int(x) for x in rng.integers(0, 200, 30)]
+    lens = [0, 1, 32, 33, most, 64] + [int(x) for x in rng.integers(0, 200, 30)]
     caches, refs = [], []
     n = len(lens)
     kn, vn, q = normal(rng, n, 2, 256), normal(rng, n, 2, 256), normal(rng, n, 16, 256)

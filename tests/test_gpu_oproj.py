@@ -135,6 +135,27 @@ def test_batched_form_matches_oracle(pk, orc, w_type, b, in_dim, out_dim, gated)
     assert rms_rel_err(out, ref) < 2e-5
 
 
+@pytest.mark.parametrize("w_type", [W_Q4K, W_Q5K, W_Q6K])
+@pytest.mark.parametrize("b,in_dim,out_dim,gated", [(383, 4096, 300, True), (384, 4096, 300, True),
+                                                    (385, 4096, 260, False), (449, 4096, 776, True),
+                                                    (400, 8192, 264, False)])
+def test_wide_tiles_match_float64(pk, orc, w_type, b, in_dim, out_dim, gated):
+    """Either side of the 384 tokens from which a workgroup takes 64: ragged last tiles of tokens
+    and of rows, both input widths, against a float64 product over the oracle's rows."""
+    from kquant_blocks import random_weight_bytes
+    say(f"oproj wide w_type={w_type} b={b} in={in_dim} out={out_dim} gated={gated}")
+    rng = np.random.default_rng(5000 * w_type + in_dim + out_dim + b)
+    wb = random_weight_bytes(rng, w_type, out_dim, in_dim, d_scale=1e-4)
+    x = rng.standard_normal((b, in_dim)).astype(np.float32)
+    g = rng.standard_normal((b, in_dim)).astype(np.float32) if gated else None
+    out = host(pk.gated_o_proj(dev(x), dev(g) if gated else None, dev(wb), out_dim, w_type=w_type))
+    wdq = orc.dequantize_weight(wb, w_type, out_dim * in_dim).reshape(out_dim, in_dim)
+    y = x.astype(np.float64)
+    if gated:
+        y = y / (1.0 + np.exp(-g.astype(np.float64)))
+    assert rms_rel_err(out, y @ wdq.astype(np.float64).T) < 2e-5
+
+
 def test_batched_form_token_scales(pk, orc):
     """Per-token power-of-two scaling: rows of 1e-30, 1e4 and 0 magnitudes beside N(0, 1)
     rows keep the relative accuracy of each row; the zero row gives exact zeros."""
