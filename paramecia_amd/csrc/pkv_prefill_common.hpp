@@ -108,11 +108,12 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(const float *part, c
 
 // The same for up to kMaxMergeSplits splits (a short chunk over many keys): one workgroup
 // of 8 groups of 32 threads per row and batch. Group sg takes splits sg, sg + 8, ...: up
-// to 16 of them, every load issued before any is used; the groups' sums meet in LDS.
+// to kPer of them, every load issued before any is used; the groups' sums meet in LDS.
+// (2 x 33 tokens over 3033 keys at 20 splits: 41.3 us with 16 loads a group, 35.4 with 4.)
+template <int kPer>
 __global__ __launch_bounds__(256) void prefill_merge_wide_kernel(const float *part,
                                                                  const float2 *pml, int nsplit,
                                                                  int l, float *out) {
-  constexpr int kPer = kMaxMergeSplits / 8;
   __shared__ __attribute__((aligned(16))) float acc_s[8][256];
   __shared__ float2 ml_s[8];
   const int sg = threadIdx.x >> 5, j = threadIdx.x & 31;
@@ -174,35 +175,45 @@ static inline size_t prefill_part_bytes(int batch, int nsplit, int l) {
 }
 
 // The number of key splits: the one with the least estimated time, in units of a block
-// (32 keys) of one workgroup, of which 256 run at a time (one per CU).
-//   rounds x (a workgroup's mean blocks + kPfFixed), or the longest workgroup's time where
-//   that is more, + the merge's time (its partials written and read once).
-// A chunk that fills the GPU by itself keeps one split; 512 tokens over 16896 keys take 4
-// (256 workgroups); a few tokens over a long cache take as many as give every CU a
-// workgroup: 5 tokens over 20016 keys ran 32 workgroups at the earlier limit of 16
-// splits, 98.8 us with the merge; at 128 splits 24.5 us. The partials take kPfMaxPartBytes
-// at most: beyond lie chunks of many rows that fill the GPU without a split.
+// (32 keys) of one workgroup, of which 256 run at a time (one per CU). A workgroup takes its
+// blocks + kPfFixed. Up to 256 workgroups end with the longest one. Of more, dispatched
+// longest first, the last round's each follow one of the round before, the two as long as
+// those at the rounds' boundary. The merge writes and reads its partials. Only splits that
+// leave no share of the last tile empty are looked at.
+// Measured with every split over 2 to 4096 tokens, 0 to 60000 cached, 1 and 2 rows of Q4K, Q8_0
+// and F16 (696 shapes): the split taken is 0.4% slower than the best one in the mean, over 10%
+// in 4 shapes. Whole rounds of mean workgroups and merges twice as dear had 1.3% and 32 (Q8_0
+// 700 tokens after 500 64.1 us at 3 splits, 72.3 at the 2 taken then). A few tokens over a
+// long cache take as many splits as give every CU a workgroup: 5 tokens over 20016 keys 98.8 us
+// at 16 splits, 24.5 at 126. The partials take kPfMaxPartBytes at most: beyond lie chunks of
+// many rows that fill the GPU without a split.
 static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk) {
-  constexpr double kPfFixed = 2.0;   // q, the first block's latency, the epilogue
-  constexpr double kMergeFixed = 1.5, kMergeBytes = 7e6;  // bytes merged in a block's time
-  const int base = ntiles * 2 * a.batch;
+  constexpr double kPfFixed = 2.5;  // q, the first block's latency, the epilogue
+  constexpr double kMergeFixed = 2.5, kMergeBytes = 8e6;  // bytes of partials in a block's time
   // blocks of the first and the last tile (the causal limit cuts the first ones')
-  double b0 = nblk, b1 = nblk;
+  int nb0 = nblk, nb1 = nblk;
   if (a.causal) {
-    auto seen = [&](int64_t keys) { return (double)((keys < a.seq_k ? keys : a.seq_k) + 31) / 32; };
-    b0 = seen(a.q_offset + (a.l < kPosPerWG ? a.l : kPosPerWG));
-    b1 = seen(a.q_offset + a.l);
+    auto seen = [&](int64_t keys) { return (int)(((keys < a.seq_k ? keys : a.seq_k) + 31) / 32); };
+    nb0 = seen(a.q_offset + (a.l < kPosPerWG ? a.l : kPosPerWG));
+    nb1 = seen(a.q_offset + a.l);
   }
-  const double mean = 0.5 * (b0 + b1);
   int best = 1;
   double best_t = 1e30;
-  for (int ns = 1; ns <= kMaxMergeSplits && ns <= (nblk > 0 ? nblk : 1); ++ns) {
+  for (int ns = 1; ns <= kMaxMergeSplits && ns <= (nb1 > 0 ? nb1 : 1); ++ns) {
     const size_t bytes = ns > 1 ? prefill_part_bytes(a.batch, ns, a.l) : 0;
     if (bytes > kPfMaxPartBytes) break;
-    const int64_t rounds = ((int64_t)base * ns + kPfTargetWGs - 1) / kPfTargetWGs;
-    const double even = rounds * (mean / ns + kPfFixed), longest = b1 / ns + kPfFixed;
-    const double t = (even > longest ? even : longest) +
-                     (ns > 1 ? kMergeFixed + 2.0 * bytes / kMergeBytes : 0.0);
+    const int share = (nb1 + ns - 1) / ns;
+    if (ns > 1 && (nb1 + share - 1) / share != ns) continue;
+    const double longest = share + kPfFixed, shortest = (nb0 + ns - 1) / ns + kPfFixed;
+    const double wgs = 2.0 * ntiles * a.batch * ns;
+    double t = longest;
+    if (wgs > kPfTargetWGs) {
+      const double full = (double)(int64_t)((wgs - 1) / kPfTargetWGs);  // rounds before the last
+      auto length = [&](double rounds) { return longest - (longest - shortest) * rounds * kPfTargetWGs / wgs; };
+      const double sum = (full - 1) * 0.5 * (longest + length(full - 1)) + 2 * length(full);
+      t = sum > t ? sum : t;
+    }
+    if (ns > 1) t += kMergeFixed + bytes / kMergeBytes;
     if (t < best_t) {
       best_t = t;
       best = ns;
@@ -227,9 +238,15 @@ static inline int prefill_merge(const PrefillArgs &d, int batch, hipStream_t s) 
   if (d.nsplit <= kNarrowSplits)
     hipLaunchKernelGGL(prefill_merge_kernel, dim3((unsigned)((2 * d.l * 8 + 7) / 8), (unsigned)batch),
                        dim3(256), 0, s, d.part, d.ml, d.nsplit, d.l, d.out);
-  else
-    hipLaunchKernelGGL(prefill_merge_wide_kernel, dim3((unsigned)(2 * d.l * 8), (unsigned)batch),
-                       dim3(256), 0, s, d.part, d.ml, d.nsplit, d.l, d.out);
+  else {
+    const auto wide = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3((unsigned)(2 * d.l * 8), (unsigned)batch), dim3(256), 0, s, d.part,
+                         d.ml, d.nsplit, d.l, d.out);
+    };
+    if (d.nsplit <= 32) wide(prefill_merge_wide_kernel<4>);
+    else if (d.nsplit <= 64) wide(prefill_merge_wide_kernel<8>);
+    else wide(prefill_merge_wide_kernel<kMaxMergeSplits / 8>);
+  }
   PKV_HIP(hipGetLastError());
   return PKV_OK;
 }

@@ -172,6 +172,14 @@ def test_prefill_full_chunk(pk, orc, quant):
     assert_attn_close(out, ref)
 
 
+@pytest.mark.parametrize("quant", QUANTS)
+@pytest.mark.parametrize("L", [12, 33, 64, 100])
+def test_prefill_wide_merges(pk, orc, L, quant):
+    """Up to 126, 42, 32 and 18 key splits: every form of the wide merge."""
+    say(f"prefill wide merge quant={quant} L={L}")
+    run_prefill(pk, orc, 8000, L, seed=900 + L, quant=quant)
+
+
 def test_prefill_partials_stay_bounded(pk):
     """A batch of chunks over long caches, which the GPU could run in 5 key splits (378 MB of
     partials): the plan's partials stay within 256 MiB, a workspace within 5 / 4 of that."""
