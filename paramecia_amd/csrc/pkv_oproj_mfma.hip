@@ -522,19 +522,28 @@ int launch_oproj_mfma(const float *attn, const float *gate, const uint8_t *w, in
     if (reinterpret_cast<uintptr_t>(p) % 16 != 0)
       return set_error(PKV_ERR_ARG, "attn, gate and the weights must be 16-byte aligned");
   const int T = batch, N = out_dim, K = in_dim;
-  // Tile: 32 tokens x 256 rows per workgroup of 4 waves (32 x 64 per wave), and from
-  // kWideTokens tokens on 64 tokens: Q4K and Q5K with 8 waves (two per SIMD, one's decoding
-  // beside the other's MFMAs), Q6K, whose two-plane operands would spill at 256 registers
-  // a wave, with 4 waves of 64 x 64. A decoded weight then feeds twice the tokens; below,
-  // the wide tile leaves CUs idle. us, narrow / wide: Q4K 130 tokens 27.1 / 30.1, 512 47.1 /
-  // 42.3, 4001 296 / 227; Q5K 4001 322 / 245; Q6K 512 65.8 / 61.7, 4001 444 / 377.
-  constexpr int kWideTokens = 384;
-  const bool wide = T >= kWideTokens;
-  const int tok = wide ? 64 : 32, rows = 256;
+  // Tile: 32 tokens x 256 rows per workgroup of 4 waves (32 x 64 per wave), or 64 tokens: Q4K
+  // and Q5K with 8 waves (two per SIMD, one's decoding beside the other's MFMAs), Q6K, whose
+  // two-plane operands would spill at 256 registers a wave, with 4 waves of 64 x 64. A decoded
+  // weight then feeds twice the tokens, but fewer than kWideWGs such workgroups have to split
+  // K so far that their epilogues and the reduction cost more: wide / narrow time of Q4K, 4096
+  // wide inputs, 8 to 24 workgroups 1.19 to 1.01, 32 1.04 to 0.98, 40 0.94, 64 0.93, 80 and more
+  // 0.90 to 0.71 (1 to 32 row blocks; Q5K and Q6K alike). Past 256 workgroups (one per CU)
+  // a wide round takes 1.5 times a narrow one, 1.7 times for Q6K, which is then wide only
+  // where that saves rounds: 288 workgroups 1.12, 512 0.84.
+  // us, narrow / wide, 4096 -> 2048: Q4K 130 tokens 27.1 / 30.1, 512 47.1 / 42.3, 4001 296 /
+  // 227; Q5K 4001 322 / 245; Q6K 512 65.8 / 61.7, 4001 444 / 377; -> 300, Q4K 400 tokens 25.1 /
+  // 29.3.
+  constexpr int kWideWGs = 40;
+  const int rows = 256, rbs = (N + rows - 1) / rows;
+  const auto wgs = [&](int tokens) { return (int64_t)rbs * ((T + tokens - 1) / tokens); };
+  bool wide = wgs(64) >= kWideWGs;
+  if (w_type == kMQ6K && wgs(64) > 256) wide = 17 * ((wgs(64) + 255) / 256) < 10 * ((wgs(32) + 255) / 256);
+  const int tok = wide ? 64 : 32;
   const int T_pad = (T + tok - 1) / tok * tok;
   const int KB = K / 32, SB = K / 256;
   const int64_t row_bytes = (int64_t)SB * (w_type == kMQ4K ? 144 : w_type == kMQ5K ? 176 : 210);
-  const int rbs = (N + rows - 1) / rows, tbs = T_pad / tok;
+  const int tbs = T_pad / tok;
   if ((int64_t)rbs * tbs * SB > (1 << 30))
     return set_error(PKV_ERR_ARG, "batch too large for the batched o_proj");
   int S = kMxTargetWGs / (rbs * tbs);

@@ -136,12 +136,13 @@ def test_batched_form_matches_oracle(pk, orc, w_type, b, in_dim, out_dim, gated)
 
 
 @pytest.mark.parametrize("w_type", [W_Q4K, W_Q5K, W_Q6K])
-@pytest.mark.parametrize("b,in_dim,out_dim,gated", [(383, 4096, 300, True), (384, 4096, 300, True),
-                                                    (385, 4096, 260, False), (449, 4096, 776, True),
-                                                    (400, 8192, 264, False)])
+@pytest.mark.parametrize("b,in_dim,out_dim,gated", [(256, 4096, 2048, True), (257, 4096, 2048, True),
+                                                    (449, 4096, 1290, False), (1217, 4096, 300, True),
+                                                    (283, 8192, 2100, False), (4161, 4096, 1030, True)])
 def test_wide_tiles_match_float64(pk, orc, w_type, b, in_dim, out_dim, gated):
-    """Either side of the 384 tokens from which a workgroup takes 64: ragged last tiles of tokens
-    and of rows, both input widths, against a float64 product over the oracle's rows."""
+    """Either side of the 40 workgroups of 64 tokens x 256 rows from which such tiles are taken,
+    ragged last tiles of tokens and of rows, both input widths, and more workgroups than CUs
+    (Q6K takes the narrow tiles then), against a float64 product over the oracle's rows."""
     from kquant_blocks import random_weight_bytes
     say(f"oproj wide w_type={w_type} b={b} in={in_dim} out={out_dim} gated={gated}")
     rng = np.random.default_rng(5000 * w_type + in_dim + out_dim + b)
