@@ -378,10 +378,10 @@ __global__ __launch_bounds__(256) void prep_tiles_kernel(PrepArgs a, uint32_t kv
     y[4 * i + 3] = t.w;
   }
   const bool live = base + rr < a.kv_rows;
-  uint8_t *dst = dst_row(live ? base + rr : a.kv_rows - 1);
   if constexpr (kFmt == kTileQ4K) {
-    q4k_quantize_group<kL>(y, r, dst, live);
+    q4k_quantize_group<kL>(y, r, [&] { return dst_row(base + rr); }, live);
   } else {  // one lane per block
+    uint8_t *dst = dst_row(live ? base + rr : a.kv_rows - 1);
     static_assert(kL == 1, "Q8_0: one lane per block");
     float amax = 0.0f;
 #pragma unroll

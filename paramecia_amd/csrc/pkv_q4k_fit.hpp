@@ -70,10 +70,11 @@ __device__ __forceinline__ bool group_any(bool c) {
 // gives the fewest instructions per superblock (large appends) and kL = 2 or 4 the
 // shortest instruction stream per wave (appends with too few superblocks to fill the GPU).
 // Cross-lane work is limited to exact moves, max reductions and byte shuffles.
-// r: the lane's index in its superblock's 8 kL (j = r / kL, s = r % kL); blk: the block's 144
-// bytes, written where `active`.
-template <int kL>
-__device__ __forceinline__ void q4k_quantize_group(const float (&x)[32 / kL], int r, uint8_t *blk,
+// r: the lane's index in its superblock's 8 kL (j = r / kL, s = r % kL); block(): the block's 144
+// bytes, written where `active` (asked for at the end: an address held through the fit cost
+// 2.7% of an append of 4096 tokens, 14.46 us against 14.08).
+template <int kL, typename Block>
+__device__ __forceinline__ void q4k_quantize_group(const float (&x)[32 / kL], int r, Block block,
                                                    bool active) {
 #pragma clang fp contract(off)
   constexpr int E = 32 / kL;
@@ -237,6 +238,7 @@ __device__ __forceinline__ void q4k_quantize_group(const float (&x)[32 / kL], in
     outw[w] = v;
   }
   if (!active) return;
+  uint8_t *const blk = block();
   uint8_t *qdst = blk + 16 + 32 * (j >> 1) + s * E + (odd ? H : 0);
   if constexpr (NB == 4) {
     *reinterpret_cast<uint4 *>(qdst) = uint4{outw[0], outw[1], outw[2], outw[3]};

@@ -57,8 +57,8 @@ __device__ __forceinline__ uint8_t *row_ptr(const AppendArgs &a, int p, int64_t 
 }
 
 // One group of 8 kL lanes per superblock (q4k_quantize_group), every superblock of K, then
-// of V.
-template <int kL>
+// of V. kWide: 16-byte loads from both tensors.
+template <int kL, bool kWide>
 __global__ __launch_bounds__(256) void q4k_append_kernel(AppendArgs a, int64_t units_per_tensor,
                                                          int nsb) {
   constexpr int E = 32 / kL;
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(256) void q4k_append_kernel(AppendArgs a, int64_t u
   float x[E];
   const int e0 = sb * 256 + 32 * j + s * E;
   const float *src = a.src[p];
-  if ((a.head_dim & 3) == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0 && e0 + E <= a.head_dim) {
+  if (kWide && e0 + E <= a.head_dim) {
     const float4 *s4 = reinterpret_cast<const float4 *>(
         src + (((int64_t)b * a.heads + h) * a.n + t) * a.head_dim + e0);
 #pragma unroll
@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void q4k_append_kernel(AppendArgs a, int64_t u
     for (int i = 0; i < E; ++i) x[i] = load_elem(src, a, t, b, h, e0 + i);
   }
 
-  q4k_quantize_group<kL>(x, r, row_ptr(a, p, t, b, h) + (int64_t)sb * 144, active);
+  q4k_quantize_group<kL>(x, r, [&] { return row_ptr(a, p, t, b, h) + (int64_t)sb * 144; }, active);
 }
 
 // Four elements of a row per lane: 16-byte loads where kWide (head_dim a multiple of 4, K
@@ -325,12 +325,10 @@ static int launch_append_args(int quant, AppendArgs &a, hipStream_t s) {
     const int kl = 2 * units <= kQ4kAppendLanes4Max ? 4 : (2 * units <= kQ4kAppendLanes2Max ? 2 : 1);
     const int64_t threads = 2 * units * 8 * kl;
     const dim3 grid((unsigned)((threads + 255) / 256));
-    if (kl == 4)
-      hipLaunchKernelGGL(q4k_append_kernel<4>, grid, dim3(256), 0, s, a, units, nsb);
-    else if (kl == 2)
-      hipLaunchKernelGGL(q4k_append_kernel<2>, grid, dim3(256), 0, s, a, units, nsb);
-    else
-      hipLaunchKernelGGL(q4k_append_kernel<1>, grid, dim3(256), 0, s, a, units, nsb);
+    const auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a, units, nsb); };
+    if (kl == 4) go(wide ? q4k_append_kernel<4, true> : q4k_append_kernel<4, false>);
+    else if (kl == 2) go(wide ? q4k_append_kernel<2, true> : q4k_append_kernel<2, false>);
+    else go(wide ? q4k_append_kernel<1, true> : q4k_append_kernel<1, false>);
   } else {
     const bool q8 = quant == PKV_QUANT_Q8_0, bf = quant == PKV_QUANT_BF16;
     const int64_t elems = rows * a.padded, blocks = (2 * (elems / 4) + 255) / 256;
