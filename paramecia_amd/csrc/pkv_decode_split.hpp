@@ -257,16 +257,19 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(CombineArgsT<kRows>
   const int b = blockIdx.y;
   combine_row(fs, c.part, c.ml, c.q, c.dq, c.out, c.sl2, c.wg0[b], c.wg1[b] - c.wg0[b], b);
 }
-// Rows of at most kCombRowMax partials (a serving batch: its 256 workgroups' partials shared
-// out over the rows): one workgroup per (head, row), 4 slices of 64 threads, thread (ps, g)
-// taking entries 4 g .. + 3 of partials ps, ps + 4, ..., all in flight at once. The form above
-// has 32 slices per 32 entries, most of them without a partial then.
-// Taken from kCombRows rows on. us after a kernel that writes the partials, form above / this
-// one, rows x partials: 6 x 8 2.8 / 3.0, 6 x 32 4.2 / 4.3 (16 workgroups a row leave the chip
-// idle); 8 x 8 3.2 / 3.2, 8 x 32 5.0 / 4.3; 16 x 4 4.4 / 3.2, 16 x 32 7.5 / 6.0; 32 x 8 7.9 /
-// 4.7, 32 x 32 12.9 / 9.5. A second round of loads (33 partials and more) does not pay at few
-// rows: 8 x 40 5.1 / 6.0, 16 x 64 10.0 / 10.4, 32 x 40 13.7 / 12.3.
-constexpr int kCombRowMax = 4 * kCombChunk, kCombRows = 8;
+// Rows of few partials (a serving batch: its 256 workgroups' partials shared out over the
+// rows): one workgroup per (head, row), 4 slices of 64 threads, thread (ps, g) taking entries
+// 4 g .. + 3 of partials ps, ps + 4, ..., 32 partials in flight at once. The form above has 32
+// slices per 32 entries, most of them without a partial then. comb_by_rows takes it where it
+// is the faster one; us after a kernel that writes the partials, form above / this one, rows x
+// partials: 6 x 8 2.8 / 3.0, 6 x 32 4.2 / 4.3 (16 workgroups a row leave the chip idle); 8 x 8
+// 3.2 / 3.2, 8 x 32 5.0 / 4.3; 16 x 4 4.4 / 3.2, 16 x 32 7.5 / 6.0; 32 x 8 7.9 / 4.7, 32 x 32
+// 12.9 / 9.5. A second round of loads pays from 16 rows on and up to 40 partials a row in the
+// mean: 8 x 40 5.1 / 6.0, 12 rows of 10 but one of 64 4.6 / 5.0; 16 x 40 7.8 / 7.4, 16 x 64 10.0
+// / 10.4, 16 rows of 10 but one of 64 5.4 / 5.3; 32 x 40 13.7 / 12.3, 32 x 64 15.5 / 16.9.
+static inline bool comb_by_rows(int n, int most, int total) {
+  return n >= 8 && (most <= 32 || (n >= 16 && most <= 64 && total <= 40 * n));
+}
 template <int kRows>
 __global__ __launch_bounds__(256) void decode_combine_rows_kernel(CombineArgsT<kRows> c) {
   __shared__ __attribute__((aligned(16))) float acc_s[4][kPartRow];
@@ -277,14 +280,17 @@ __global__ __launch_bounds__(256) void decode_combine_rows_kernel(CombineArgsT<k
   const float2 *ML = c.ml + (int64_t)wbeg * 16 + h;
   float2 mlv[kCombChunk];
   float4 ov[kCombChunk];
+  auto load_round = [&](int w) {  // past the partials: the first one's, with no weight
 #pragma unroll
-  for (int x = 0; x < kCombChunk; ++x) {  // past the partials: the first one's, with no weight
-    const bool ok = ps + 4 * x < np;
-    const int64_t i = ok ? ps + 4 * x : 0;
-    const float2 t = ML[i * 16];
-    ov[x] = *reinterpret_cast<const float4 *>(P + i * 16 * kPartRow);
-    mlv[x] = ok ? t : float2{-INFINITY, 0.0f};
-  }
+    for (int x = 0; x < kCombChunk; ++x) {
+      const bool ok = w + 4 * x < np;
+      const int64_t i = ok ? w + 4 * x : 0;
+      const float2 t = ML[i * 16];
+      ov[x] = *reinterpret_cast<const float4 *>(P + i * 16 * kPartRow);
+      mlv[x] = ok ? t : float2{-INFINITY, 0.0f};
+    }
+  };
+  load_round(ps);
   const int e = tile_e(tid >> 4, tid & 15);
   const bool has_new = c.dq != nullptr;
   float qk = 0.0f, vnew = 0.0f;
@@ -294,17 +300,29 @@ __global__ __launch_bounds__(256) void decode_combine_rows_kernel(CombineArgsT<k
   }
   float m = -INFINITY, l = 0.0f;
   float4 acc = {0.f, 0.f, 0.f, 0.f};
+  for (int w = ps; w < np; w += 4 * kCombChunk) {
+    if (w != ps) load_round(w);
+    float mc = m;
 #pragma unroll
-  for (int x = 0; x < kCombChunk; ++x) m = fmaxf(m, mlv[x].x);
+    for (int x = 0; x < kCombChunk; ++x) mc = fmaxf(mc, mlv[x].x);
+    if (mc == -INFINITY) continue;
+    const float r = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mc);
+    acc.x *= r;
+    acc.y *= r;
+    acc.z *= r;
+    acc.w *= r;
+    l *= r;
 #pragma unroll
-  for (int x = 0; x < kCombChunk; ++x) {
-    if (mlv[x].x == -INFINITY) continue;
-    const float f = __builtin_amdgcn_exp2f(mlv[x].x - m);
-    acc.x += f * ov[x].x;
-    acc.y += f * ov[x].y;
-    acc.z += f * ov[x].z;
-    acc.w += f * ov[x].w;
-    l += f * mlv[x].y;
+    for (int x = 0; x < kCombChunk; ++x) {
+      if (mlv[x].x == -INFINITY) continue;
+      const float f = __builtin_amdgcn_exp2f(mlv[x].x - mc);
+      acc.x += f * ov[x].x;
+      acc.y += f * ov[x].y;
+      acc.z += f * ov[x].z;
+      acc.w += f * ov[x].w;
+      l += f * mlv[x].y;
+    }
+    m = mc;
   }
   const float d = wave_sum(qk);
   *reinterpret_cast<float4 *>(&acc_s[ps][4 * g]) = acc;
@@ -561,7 +579,7 @@ static inline int launch_combine(const CombineArgs &c, int n, hipStream_t s) {
   } else {
     int most = 0;
     for (int i = 0; i < n; ++i) most = c.wg1[i] - c.wg0[i] > most ? c.wg1[i] - c.wg0[i] : most;
-    if (n >= kCombRows && most <= kCombRowMax)
+    if (comb_by_rows(n, most, c.wg1[n - 1] - c.wg0[0]))
       hipLaunchKernelGGL(decode_combine_rows_kernel<kMaxSegs>, dim3(16, (unsigned)n), dim3(256), 0,
                          s, c);
     else

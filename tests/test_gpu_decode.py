@@ -415,11 +415,13 @@ def test_q8_decode_without_mfma():
     assert r.returncode == 0
 
 
-@pytest.mark.parametrize("lens", [[1024] * 7 + [5], [1025] + [40] * 7, [1024] * 7, [992, 1, 0, 33] * 8],
-                         ids=["8x32", "8x33", "7x32", "32x31"])
+@pytest.mark.parametrize("lens", [[1024] * 7 + [5], [1025] + [40] * 7, [1024] * 7, [992, 1, 0, 33] * 8,
+                                  [2048] + [33] * 15, [2049] + [33] * 15, [1280] * 15 + [1313]],
+                         ids=["8x32", "8x33", "7x32", "32x31", "16x64", "16x65", "16x40"])
 def test_combine_forms(pk, orc, lens):
     """A Q8_0 sequence has one partial per 32 keys: rows and partials on either side of where
-    the combine with one workgroup per head and row is taken (8 rows, 32 partials)."""
+    the combine with one workgroup per head and row is taken (8 rows of 32 partials, 16 of 64, 40
+    in the mean)."""
     say(f"combine of {len(lens)} rows of up to {max(lens)} keys")
     run_batched(pk, orc, lens, seed=len(lens), quant=Q8_0)
 
