@@ -189,7 +189,8 @@ static inline size_t prefill_part_bytes(int batch, int nsplit, int l) {
 // many rows that fill the GPU without a split.
 static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk) {
   constexpr double kPfFixed = 2.5;  // q, the first block's latency, the epilogue
-  constexpr double kMergeFixed = 2.5, kMergeBytes = 8e6;  // bytes of partials in a block's time
+  // bytes of partials in a block's time; twice the time for those past kMergeNear
+  constexpr double kMergeFixed = 2.5, kMergeBytes = 8e6, kMergeNear = 64e6;
   // blocks of the first and the last tile (the causal limit cuts the first ones')
   int nb0 = nblk, nb1 = nblk;
   if (a.causal) {
@@ -213,7 +214,7 @@ static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk) {
       const double sum = (full - 1) * 0.5 * (longest + length(full - 1)) + 2 * length(full);
       t = sum > t ? sum : t;
     }
-    if (ns > 1) t += kMergeFixed + bytes / kMergeBytes;
+    if (ns > 1) t += kMergeFixed + (bytes + (bytes > kMergeNear ? bytes - kMergeNear : 0.0)) / kMergeBytes;
     if (t < best_t) {
       best_t = t;
       best = ns;
