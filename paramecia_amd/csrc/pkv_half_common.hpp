@@ -74,6 +74,48 @@ __device__ __forceinline__ T row_load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
     return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
 }
 
+// kH heads (q rows of 256 floats) over keys [j0, j1) in f32 products, element for element what the
+// general kernel (pkv_attn.hip) computes: lane owns elements 4 lane .. + 3; m in log2 units. A
+// key's rows are read once for all heads (5 tokens over 20000 keys with NaN: 970 us a head at
+// a time, 300 so; the general kernel 570).
+template <int kH>
+__device__ __forceinline__ void half_slow_keys(const uint8_t *kbase, const uint8_t *vbase,
+                                               int64_t rs_t, int64_t j0, int64_t j1, const float *q,
+                                               float sl2, bool bf, int lane, float (&m)[kH],
+                                               float (&l)[kH], float (&acc)[kH][4]) {
+  float4 q4[kH];
+#pragma unroll
+  for (int h = 0; h < kH; ++h) {
+    q4[h] = reinterpret_cast<const float4 *>(q + h * 256)[lane];
+    m[h] = -INFINITY;
+    l[h] = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc[h][k] = 0.0f;
+  }
+  for (int64_t j = j0; j < j1; ++j) {
+    const uint2 kw = *reinterpret_cast<const uint2 *>(kbase + j * rs_t + 8 * lane);
+    const uint2 vw = *reinterpret_cast<const uint2 *>(vbase + j * rs_t + 8 * lane);
+    const float kf[4] = {half_value((uint16_t)kw.x, bf), half_value((uint16_t)(kw.x >> 16), bf),
+                         half_value((uint16_t)kw.y, bf), half_value((uint16_t)(kw.y >> 16), bf)};
+    const float vf[4] = {half_value((uint16_t)vw.x, bf), half_value((uint16_t)(vw.x >> 16), bf),
+                         half_value((uint16_t)vw.y, bf), half_value((uint16_t)(vw.y >> 16), bf)};
+#pragma unroll
+    for (int h = 0; h < kH; ++h) {
+      float dot = q4[h].x * kf[0];
+      dot += q4[h].y * kf[1];
+      dot += q4[h].z * kf[2];
+      dot += q4[h].w * kf[3];
+      const float s = fminf(fmaxf(wave_sum(dot) * sl2, -kClampL2), kClampL2);
+      const float mn = fmaxf(m[h], s);
+      const float c = __builtin_amdgcn_exp2f(m[h] - mn), p = __builtin_amdgcn_exp2f(s - mn);
+      l[h] = l[h] * c + p;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) acc[h][k] = acc[h][k] * c + p * vf[k];
+      m[h] = mn;
+    }
+  }
+}
+
 inline bool half_shape(int quant, int num_heads, int num_kv_heads, int head_dim) {
   return (quant == PKV_QUANT_F16 || quant == PKV_QUANT_BF16) && head_dim == 256 &&
          num_heads == 16 && num_kv_heads == 2;

@@ -69,35 +69,19 @@ struct HalfSmem {
 };
 
 // Heads h0 and h0 + 1 of a workgroup's blocks [b0, b1) in f32 products (see the header),
-// stored as its partial: lane owns elements 4 lane .. + 3.
+// stored as its partial.
 __device__ __forceinline__ void slow_heads(const uint8_t *kbase, const uint8_t *vbase,
                                            int64_t rs_t, int64_t seq_k, int b0, int b1,
                                            const float *q, int h0, float sl2, bool bf, int lane,
                                            float *part, float2 *ml) {
-  for (int h = h0; h < h0 + 2; ++h) {
-    const float4 q4 = reinterpret_cast<const float4 *>(q + h * 256)[lane];
-    float m = -INFINITY, l = 0.0f, acc[4] = {0.f, 0.f, 0.f, 0.f};
-    const int64_t k1 = (int64_t)b1 * kBlk < seq_k ? (int64_t)b1 * kBlk : seq_k;
-    for (int64_t j = (int64_t)b0 * kBlk; j < k1; ++j) {
-      const uint2 kw = *reinterpret_cast<const uint2 *>(kbase + j * rs_t + 8 * lane);
-      const uint2 vw = *reinterpret_cast<const uint2 *>(vbase + j * rs_t + 8 * lane);
-      float dot = q4.x * half_value((uint16_t)kw.x, bf);
-      dot += q4.y * half_value((uint16_t)(kw.x >> 16), bf);
-      dot += q4.z * half_value((uint16_t)kw.y, bf);
-      dot += q4.w * half_value((uint16_t)(kw.y >> 16), bf);
-      const float s = fminf(fmaxf(wave_sum(dot) * sl2, -kClampL2), kClampL2);
-      const float mn = fmaxf(m, s);
-      const float c = __builtin_amdgcn_exp2f(m - mn), p = __builtin_amdgcn_exp2f(s - mn);
-      l = l * c + p;
-      acc[0] = acc[0] * c + p * half_value((uint16_t)vw.x, bf);
-      acc[1] = acc[1] * c + p * half_value((uint16_t)(vw.x >> 16), bf);
-      acc[2] = acc[2] * c + p * half_value((uint16_t)vw.y, bf);
-      acc[3] = acc[3] * c + p * half_value((uint16_t)(vw.y >> 16), bf);
-      m = mn;
-    }
+  const int64_t k1 = (int64_t)b1 * kBlk < seq_k ? (int64_t)b1 * kBlk : seq_k;
+  float m[2], l[2], acc[2][4];
+  half_slow_keys<2>(kbase, vbase, rs_t, (int64_t)b0 * kBlk, k1, q + h0 * 256, sl2, bf, lane, m, l, acc);
 #pragma unroll
-    for (int k = 0; k < 4; ++k) part[h * kPartRow + tile_index(4 * lane + k)] = acc[k];
-    if (lane == 0) ml[h] = float2{m, l};
+  for (int x = 0; x < 2; ++x) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) part[(h0 + x) * kPartRow + tile_index(4 * lane + k)] = acc[x][k];
+    if (lane == 0) ml[h0 + x] = float2{m[x], l[x]};
   }
 }
 

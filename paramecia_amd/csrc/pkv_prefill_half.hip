@@ -36,45 +36,29 @@ struct HalfPfSmem {
   HalfBlock blk[2];  // block i in blk[i & 1] while block i + 1 is written
 };
 
-// A wave's rows (positions pw, pw + 1) over keys [k0, k1) in f32 products: lane owns
-// elements 4 lane .. + 3. Writes the rows' outputs or partials.
+// A wave's rows (positions pw, pw + 1) over keys [k0, k1) in f32 products. Writes the rows'
+// outputs or partials.
 __device__ __forceinline__ void slow_wave(const PrefillArgs &a, const uint8_t *kbase,
                                           const uint8_t *vbase, int64_t k0, int64_t k1, int pw,
                                           int b, int kvg, int64_t r0, bool bf, int lane) {
-  for (int row = 0; row < 16; ++row) {
-    const int pos = pw + (row >> 3);
-    if (pos >= a.l) return;
-    const int64_t qr = ((int64_t)b * a.l + pos) * 16 + 8 * kvg + (row & 7);
-    const float4 q4 = reinterpret_cast<const float4 *>(a.q + qr * 256)[lane];
+  for (int pos = pw; pos < pw + 2 && pos < a.l; ++pos) {
+    const int64_t qr = ((int64_t)b * a.l + pos) * 16 + 8 * kvg;
     const int64_t lim = a.causal ? pos + a.q_offset + 1 : a.seq_k;
-    const int64_t kend = lim < k1 ? lim : k1;
-    float m = -INFINITY, l = 0.0f, acc[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int64_t j = k0; j < kend; ++j) {
-      const uint2 kw = *reinterpret_cast<const uint2 *>(kbase + j * a.rs_t + 8 * lane);
-      const uint2 vw = *reinterpret_cast<const uint2 *>(vbase + j * a.rs_t + 8 * lane);
-      float dot = q4.x * half_value((uint16_t)kw.x, bf);
-      dot += q4.y * half_value((uint16_t)(kw.x >> 16), bf);
-      dot += q4.z * half_value((uint16_t)kw.y, bf);
-      dot += q4.w * half_value((uint16_t)(kw.y >> 16), bf);
-      const float s = fminf(fmaxf(wave_sum(dot) * a.sl2, -kClampL2), kClampL2);
-      const float mn = fmaxf(m, s);
-      const float c = __builtin_amdgcn_exp2f(m - mn), p = __builtin_amdgcn_exp2f(s - mn);
-      l = l * c + p;
-      acc[0] = acc[0] * c + p * half_value((uint16_t)vw.x, bf);
-      acc[1] = acc[1] * c + p * half_value((uint16_t)(vw.x >> 16), bf);
-      acc[2] = acc[2] * c + p * half_value((uint16_t)vw.y, bf);
-      acc[3] = acc[3] * c + p * half_value((uint16_t)(vw.y >> 16), bf);
-      m = mn;
-    }
-    if (a.nsplit == 1) {
-      const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    float m[8], l[8], acc[8][4];
+    half_slow_keys<8>(kbase, vbase, a.rs_t, k0, lim < k1 ? lim : k1, a.q + qr * 256, a.sl2, bf, lane,
+                      m, l, acc);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) a.out[qr * 256 + 4 * lane + k] = acc[k] * inv;
-    } else {
-      const int64_t r = r0 + (int64_t)pos * 8 + (row & 7);
+    for (int h = 0; h < 8; ++h) {
+      if (a.nsplit == 1) {
+        const float inv = l[h] > 0.0f ? 1.0f / l[h] : 0.0f;
 #pragma unroll
-      for (int k = 0; k < 4; ++k) a.part[r * 256 + tile_index(4 * lane + k)] = acc[k];
-      if (lane == 0) a.ml[r] = float2{m, l};
+        for (int k = 0; k < 4; ++k) a.out[(qr + h) * 256 + 4 * lane + k] = acc[h][k] * inv;
+      } else {
+        const int64_t r = r0 + (int64_t)pos * 8 + h;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) a.part[r * 256 + tile_index(4 * lane + k)] = acc[h][k];
+        if (lane == 0) a.ml[r] = float2{m[h], l[h]};
+      }
     }
   }
 }
