@@ -1166,7 +1166,7 @@ int pkv_deltanet_step(const float *q, const float *k, const float *v, const floa
 }
 
 // From this many tokens on, the k-quant projection runs as the batched MFMA form (each
-// decoded weight serves 32 tokens); below it, per-token GEMV workgroups.
+// decoded weight serves 32 or 64 tokens); below it, per-token GEMV workgroups.
 constexpr int kOprojMfmaMinBatch = 8;
 
 int pkv_gated_oproj(const float *attn, const float *gate, const void *w, int w_type, float *out,

@@ -31,7 +31,7 @@
 //
 // Infinities and NaN (a float cache stores what it is given; F16 overflows to infinity):
 // a split operand times infinity can give inf - inf, so a wave whose scores or sums come
-// out non-finite redoes its blocks in plain f32 products (slow_rows), element for element
+// out non-finite redoes its blocks in plain f32 products (slow_heads), element for element
 // what the general kernel (pkv_attn.hip) computes.
 #include "pkv_decode_split.hpp"
 #include "pkv_half_common.hpp"

@@ -282,12 +282,12 @@ __device__ __forceinline__ float xsum32(float x) {  // x of lanes l and l ^ 32, 
   return __builtin_bit_cast(float, r0) + __builtin_bit_cast(float, r1);
 }
 
-
-}  // namespace
 // LDS written before is visible to the workgroup after; loads from memory stay in flight.
 __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
+
+}  // namespace
 }  // namespace pkv

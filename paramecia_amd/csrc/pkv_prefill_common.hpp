@@ -1,8 +1,8 @@
-// Shared parts of the MFMA prefill-chunk kernels (Q4K and Q8_0 caches, the Qwen3-Next
-// full-attention shape: 16 query heads, 2 KV heads, head_dim 256): the kernel arguments,
-// the work plan (16 query positions x one KV head x one key split per workgroup, splits
-// chosen to fill about 256 workgroups) and the kernel that merges the key splits' (m, l,
-// o) partials. Include-only; every symbol has internal linkage.
+// Shared parts of the MFMA prefill-chunk kernels (Q4K, Q8_0, F16 and BF16 caches, the
+// Qwen3-Next full-attention shape: 16 query heads, 2 KV heads, head_dim 256): the kernel
+// arguments, the work plan (16 query positions x one KV head x one key split per workgroup,
+// up to 128 splits by estimated time) and the kernels that merge the key splits' (m, l, o)
+// partials. Include-only; every symbol has internal linkage.
 //
 // Partial layout: part[batch * nsplit + split][kv head][pos * 8 + head of the group][256] in
 // tile order (entry i holds element tile_e(i / 16, i % 16)), and ml[same rows]: the row's

@@ -188,8 +188,8 @@ __global__ __launch_bounds__(kPrepThreads) void prep_append_kernel(PrepArgs a, i
 // ---- many rows (head_dim 256): tiles of rows per workgroup
 //
 // The row kernel above has one lane add a row's 256 squares in order while the other 63
-// (a K row: 255) wait, and quantizes a K or V row as one latency chain: 145 us for 4001
-// tokens, of which the bytes (147 MB) take about 30 at the copy rate. Here a workgroup takes a tile of rows
+// (a K row: 255) wait, and quantizes a K or V row as one latency chain: 136 us for 4001
+// tokens of Q4K, of which the bytes (147 MB) take about 30 at the copy rate. Here a workgroup takes a tile of rows
 // of one kind; the squares of the tile go to LDS and lane r adds those of row r, so the
 // ordered sums of all its rows run side by side; the normalised rows are quantized with 8
 // kL lanes per row, as pkv_append does (kL from the row count, by the same limits).

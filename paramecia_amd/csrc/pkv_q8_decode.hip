@@ -361,7 +361,7 @@ __device__ __forceinline__ void q8_v_codes_dec(const uint32_t (*rows)[kQ8RowWord
 // loads of a one-segment launch wait for no kernel-argument fetch.
 // kForm: kQ8Many, more than one block per workgroup. The next block's rows are loaded while this
 // one is worked on (the barriers wait for LDS only), in at most 128 registers so that two
-// workgroups still share a CU: 32768 keys 19.75 to 18.46 us, attend alone. kQ8Full, one block
+// workgroups still share a CU: 32768 keys 20.1 to 19.2 us a step. kQ8Full, one block
 // and two workgroups per CU or more: as straight code, which the compiler puts into 56
 // registers, so that four share a CU. kQ8Few, one block and fewer workgroups: compiled as a
 // loop, with its loads and LDS reads issued earlier in 122 registers. us per step, kQ8Few /
@@ -702,8 +702,8 @@ static int launch_q8_segments(const DecodeSegIn *in, int n, const float *q, cons
   d.wps = 0;
   // The MFMA kernel for caches in the standard row layout (both heads' 272-byte rows
   // adjacent, 16-byte aligned): 32-key blocks, up to 256 workgroups per KV head and segment
-  // (attend of 40000 / 65536 / 131072 keys: VALU kernel 35.8 / 45.9 / 81.5 us, MFMA 21.5 /
-  // 29.3 / 50.4). Otherwise the VALU kernel: one chunk per workgroup while that keeps <= 512
+  // (step of 40000 / 65536 / 131072 keys: VALU kernel 36.3 / 48.0 / 86.2 us, MFMA 22.4 /
+  // 31.2 / 54.1). Otherwise the VALU kernel: one chunk per workgroup while that keeps <= 512
   // partials per segment (16-key chunks up to 8192 keys, 32-key chunks beyond), more chunks
   // per workgroup for longer caches.
   bool mfma = rs_h == kQ8Row && rs_t % 16 == 0 && rs_t < (1 << 24) &&
