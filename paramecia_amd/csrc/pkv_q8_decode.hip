@@ -287,19 +287,19 @@ __global__ __launch_bounds__(kQ8Threads) void q8_decode_kernel(Q8Args a) {
 // (lo remainder): one MFMA per tile, rows h and h + 8 summed at the end. The partial goes
 // out in tile order, as the other decode kernels write it, for decode_combine_kernel.
 //
-// Both pairs are split at a power of two of their own, undone in f32: 32 q values of a head at
-// their largest, the weights at the largest d_j of the wave's keys so far. A value's hi + lo
+// Both pairs are split at a power of two of their own, undone in f32: a head's q at its
+// largest value, the weights at the largest d_j of the wave's keys so far. A value's hi + lo
 // is then off by 2^-23 of it, or 2^-40 of that largest one. Split as they are, a weight was
 // off by 2^-25 however small V is and |q| >= 65520 became infinite. Relative error against 64
 // bits, N(0, 1) rows: 4096 keys 3.7e-6 (V times 1e-3: 3.7e-3), now 1.7e-7 (1.7e-7); 131072
 // keys 7.2e-6 (7.3e-3), now 2.5e-7 (2.4e-7), the f32 products of the VALU kernel 3.7e-7.
-// Step, us: 4096 keys 7.7 to 7.8, 32768 19.1 to 19.7, 131072 52.5 to 54.1 (VALU 86). As three
-// bf16 parts (exact) in two MFMAs each: 8.0, 20.7, 60.1.
+// Step, us: 100 keys 7.33 to 7.21, 4000 7.85 to 7.93, 32768 19.2 to 19.8, 131072 52.9 to 54.9
+// (VALU 86). As three bf16 parts (exact) in two MFMAs each: 8.0 at 4096, 20.7, 60.1.
 constexpr int kQ8mThreads = 512;
 constexpr int kVeMin = -24, kVeMax = 15;  // exponents of fp16 values
 struct Q8mSmem {
-  h8 qf[8][64];                      // QK B operands: [block j][lane]
-  float qs[8][8];                    // [block j][head]: the power of two to undo
+  u4 qf[8][64];                      // QK B operands: [block j][lane (n ^ 4 g ^ 2 (j % 2), g)]
+  float qs[8];                       // [head]: the power of two to undo
   uint32_t raw[2][32][kQ8RowWords];  // [K / V][key][row]
   float kd[8][32];                   // [block j][key]: K's d_j * sl2 (written when staged)
   float vd[8][32];                   // [block j][key]: V's d_j (written when staged)
@@ -313,6 +313,48 @@ static inline bool q8_mfma_enabled() {
     return !(e && e[0] == '0');
   }();
   return on;
+}
+
+// {fp16(a0 f), fp16(a1 f)} and, c0 and c1 the fp16 halves of cw, {fp16(a0 f - c0), fp16(a1 f -
+// c1)}, each rounded once (v_fma_mix; f is a power of two, so the products are exact). kMfma:
+// an MFMA reads the words: the wait states after fp16_sub2 (pkv_mfma_common.hpp).
+__device__ __forceinline__ uint32_t fp16_mul2(float a0, float a1, float f) {
+  uint32_t d;
+  asm("v_fma_mixlo_f16 %0, %1, %3, 0 op_sel_hi:[0,0,0]\n\t"
+      "v_fma_mixhi_f16 %0, %2, %3, 0 op_sel_hi:[0,0,0]"
+      : "=&v"(d)
+      : "v"(a0), "v"(a1), "v"(f));
+  return d;
+}
+template <bool kMfma>
+__device__ __forceinline__ uint32_t fp16_mulsub2(float a0, float a1, float f, uint32_t cw) {
+  uint32_t d;
+  if constexpr (kMfma)
+    asm("v_fma_mixlo_f16 %0, %1, %4, -%3 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %0, %2, %4, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]\n\t"
+        "s_nop 4"
+        : "=&v"(d)
+        : "v"(a0), "v"(a1), "v"(cw), "v"(f));
+  else
+    asm("v_fma_mixlo_f16 %0, %1, %4, -%3 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %0, %2, %4, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+        : "=&v"(d)
+        : "v"(a0), "v"(a1), "v"(cw), "v"(f));
+  return d;
+}
+__device__ __forceinline__ float pow2(int e) { return u2f((uint32_t)(127 + e) << 23); }  // e in [-126, 127]
+
+template <int kCtrl>
+__device__ __forceinline__ float max_dpp(float x) {
+  return fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), kCtrl,
+                                                                     0xF, 0xF, false)));
+}
+__device__ __forceinline__ float halfwave_max(float x) {  // over the 32 lanes of a wave's half
+  x = max_dpp<0xB1>(x);   // quad_perm [1, 0, 3, 2]
+  x = max_dpp<0x4E>(x);   // quad_perm [2, 3, 0, 1]
+  x = max_dpp<0x141>(x);  // row_half_mirror
+  x = max_dpp<0x140>(x);  // row_mirror
+  return xmax16(x);
 }
 
 __device__ __forceinline__ float xsum16(float x) {  // x of lanes l and l ^ 16, summed
@@ -445,39 +487,39 @@ __global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_deco
   };
   // ---- q of the head group as QK B operands, built once: fragment (j, lane (n, g)) holds
   // elements 32 j + 8 g .. + 7 of head 8 kv + n % 8, as the fp16 hi part (n < 8) or the
-  // lo remainder (n >= 8); thread t = 32 j + 8 g + h loads those of head h once and builds
-  // both fragments
+  // lo remainder (n >= 8). Half h of wave w takes head 2 w + h, lane l of it elements 8 l ..
+  // + 7, so that a head's largest value is a reduction within a half; the fragments' columns
+  // are swizzled so that 8 lanes' stores fall on all banks.
   {
-    const int tq = tid & 255, j = tq >> 5, gq = (tq >> 3) & 3, hq = tq & 7;
-    const float *qrow = q + ((int64_t)qi * 16 + 8 * kv + hq) * 256 + 32 * j + 8 * gq;
+    const int tq = tid & 255, hq = tq >> 5, piece = tq & 31, j = piece >> 2, gq = piece & 3;
+    const float *qrow = q + ((int64_t)qi * 16 + 8 * kv + hq) * 256 + 8 * piece;
     const float4 q0 = *reinterpret_cast<const float4 *>(qrow);  // threads >= 256 load again
     const float4 q1 = *reinterpret_cast<const float4 *>(qrow + 4);
     if (k0 < k1) load_block(k0, (int)(k1 - k0 < kBlk ? k1 - k0 : kBlk));
-    if (tid < 256) {  // lanes l, l ^ 8 and l ^ 16 hold a head's 32 elements of block j
-      float v8[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
+    if (tid < 256) {
+      const float v8[8] = {q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w};
       float mx = 0.0f;
 #pragma unroll
       for (int k = 0; k < 8; ++k) mx = fmaxf(mx, fabsf(v8[k]));
-      mx = xmax16(fmaxf(mx, ror8(mx)));
+      mx = halfwave_max(mx);
       int e = (int)(f2u(mx) >> 23) - 127;
       e = e < -100 ? -100 : e > 127 ? 127 : e;
-      const float f = __builtin_ldexpf(1.0f, 14 - e);
-      if (gq == 0) sm.qs[j][hq] = __builtin_ldexpf(1.0f, e - 14);
-      h8 fh, fl;
+      const float f = pow2(14 - e);
+      if (piece == 0) sm.qs[hq] = pow2(e - 14);
+      uint32_t hw[4], lw[4];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const float x = v8[k] * f;
-        const _Float16 hi = (_Float16)x;
-        fh[k] = hi;
-        fl[k] = (_Float16)(x - (float)hi);
+      for (int k = 0; k < 4; ++k) {
+        hw[k] = fp16_mul2(v8[2 * k], v8[2 * k + 1], f);
+        lw[k] = fp16_mulsub2<false>(v8[2 * k], v8[2 * k + 1], f, hw[k]);
       }
       if (__any(mx == INFINITY)) {  // an infinity is its hi part alone (inf - inf is NaN)
 #pragma unroll
         for (int k = 0; k < 8; ++k)
-          if (fabsf(v8[k]) == INFINITY) fl[k] = (_Float16)0.0f;
+          if (fabsf(v8[k]) == INFINITY) lw[k >> 1] &= (k & 1) ? 0x0000FFFFu : 0xFFFF0000u;
       }
-      sm.qf[j][16 * gq + hq] = fh;
-      sm.qf[j][16 * gq + 8 + hq] = fl;
+      const int sw = (4 * gq) ^ (2 * (j & 1));
+      sm.qf[j][16 * gq + (hq ^ sw)] = u4{hw[0], hw[1], hw[2], hw[3]};
+      sm.qf[j][16 * gq + ((8 + hq) ^ sw)] = u4{lw[0], lw[1], lw[2], lw[3]};
     }
   }
 
@@ -486,7 +528,9 @@ __global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_deco
   f4 acc[2];
 #pragma unroll
   for (int x = 0; x < 2; ++x) acc[x] = f4{0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.0f;  // head n % 8 (the same in lanes n, n ^ 8 and every g)
+  // head n % 8 (the same in lanes n, n ^ 8 and every g); the scores and m_run are in units of
+  // log2 / back
+  float m_run = -INFINITY, l_run = 0.0f, back = 1.0f;
   int ve = kVeMin;  // the weights' d_j enter times 2^(14 - ve), ve the exponent of the largest
 
   const auto sync = [] {
@@ -504,7 +548,9 @@ __global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_deco
     // (r, g): key q8_key(r, tw), elements 32 j + 8 g .. + 7)
     f4 cq[2];
     {
-      const h8 qb0 = sm.qf[2 * qd][lane], qb1 = sm.qf[2 * qd + 1][lane];
+      const h8 qb0 = __builtin_bit_cast(h8, sm.qf[2 * qd][16 * g + (n ^ (4 * g))]);
+      const h8 qb1 = __builtin_bit_cast(h8, sm.qf[2 * qd + 1][16 * g + (n ^ (4 * g) ^ 2)]);
+      back = sm.qs[n & 7];
       const uint32_t *row = &sm.raw[0][q8_key(n, tw)][0];
       const int w0i = (68 * qd + 2 + 8 * g) >> 2;  // block 2 qd: two bytes past w0i
       uint32_t x[5];
@@ -539,14 +585,14 @@ __global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_deco
     const bool vinf = de > kVeMax;
     const int ve_new = de > kVeMax ? kVeMax : de > ve ? de : ve;
     if (ve_new > ve) {
-      const float down = __builtin_ldexpf(1.0f, ve - ve_new);
+      const float down = pow2(ve - ve_new);
 #pragma unroll
       for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc[x][i] *= down;
       ve = ve_new;
     }
-    const float vf = __builtin_ldexpf(1.0f, 14 - ve);
+    const float vf = pow2(14 - ve);
     // this wave's part of its tile's scores, the columns of a head (lanes n and n ^ 8) added
     // and scaled by its keys' d_j, to LDS
     {
@@ -554,11 +600,10 @@ __global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_deco
 #pragma unroll
       for (int jj = 0; jj < 2; ++jj) {
         const float4 dk = *reinterpret_cast<const float4 *>(&sm.kd[2 * qd + jj][8 * g + 4 * tw]);
-        const float back = sm.qs[2 * qd + jj][n & 7];
-        part.x = fmaf(dk.x, (cq[jj][0] + ror8(cq[jj][0])) * back, part.x);
-        part.y = fmaf(dk.y, (cq[jj][1] + ror8(cq[jj][1])) * back, part.y);
-        part.z = fmaf(dk.z, (cq[jj][2] + ror8(cq[jj][2])) * back, part.z);
-        part.w = fmaf(dk.w, (cq[jj][3] + ror8(cq[jj][3])) * back, part.w);
+        part.x = fmaf(dk.x, cq[jj][0] + ror8(cq[jj][0]), part.x);
+        part.y = fmaf(dk.y, cq[jj][1] + ror8(cq[jj][1]), part.y);
+        part.z = fmaf(dk.z, cq[jj][2] + ror8(cq[jj][2]), part.z);
+        part.w = fmaf(dk.w, cq[jj][3] + ror8(cq[jj][3]), part.w);
       }
       sm.sp[wv][lane] = part;
     }
@@ -587,8 +632,9 @@ __global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_deco
       sc[4 * t + 2] = tot.z;
       sc[4 * t + 3] = tot.w;
     }
+    const float clamp = kSplitClampL2 * u2f(0x7F000000u - f2u(back));  // / back, a power of two
 #pragma unroll
-    for (int k = 0; k < 8; ++k) sc[k] = fminf(fmaxf(sc[k], -kSplitClampL2), kSplitClampL2);
+    for (int k = 0; k < 8; ++k) sc[k] = __builtin_amdgcn_fmed3f(sc[k], -clamp, clamp);  // (NaN: -clamp)
     if (nk < kBlk) {  // keys past the range
 #pragma unroll
       for (int k = 0; k < 8; ++k)
@@ -603,7 +649,7 @@ __global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_deco
     // some head's max rose after the first block: rescale its sums (rows by head; on the
     // first block they are still 0)
     if (c0 != k0 && __any(m_new != m_run)) {
-      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * back);
       l_run *= alpha;
       // row 4 g + i is head (4 g + i) % 8, whose alpha lane (4 g + i) % 8 holds
       const auto lane_alpha = [&](int k) {
@@ -622,10 +668,11 @@ __global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_deco
         for (int i = 0; i < 4; ++i) acc[x][i] *= ai[i];
     }
     m_run = m_new;
+    const float nm = -(m_run * back);
     float p[8];
 #pragma unroll
     for (int k = 0; k < 8; ++k) {  // (m_run is finite: a block holds a key)
-      p[k] = __builtin_amdgcn_exp2f(sc[k] - m_run);
+      p[k] = __builtin_amdgcn_exp2f(fmaf(sc[k], back, nm));
       l_run += p[k];
     }
     // A rows: n < 8 the fp16 hi parts of head n's weights times d_j of their keys, n >= 8
@@ -656,7 +703,7 @@ __global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_deco
   // stores: the combine launch reads them from another XCD's L2 misses anyway, and the
   // launch's end then has fewer dirty lines to write back.
   float *P = part + (int64_t)slot * 16 * kPartRow;
-  const float vback = __builtin_ldexpf(1.0f, ve - 14);
+  const float vback = pow2(ve - 14);
   float r[2][4];
 #pragma unroll
   for (int x = 0; x < 2; ++x)
@@ -675,7 +722,7 @@ __global__ __launch_bounds__(kQ8mThreads, kForm == kQ8Many ? 4 : 2) void q8_deco
   lt = xsum32(lt);
   if (wv == 0 && g == 0 && n < 8) {
     float *mlo = reinterpret_cast<float *>(mlb + ((int64_t)slot * 16 + 8 * kv + n));
-    store_sc1(mlo, m_run);
+    store_sc1(mlo, m_run * back);
     store_sc1(mlo + 1, lt);
   }
 }
