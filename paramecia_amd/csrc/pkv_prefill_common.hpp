@@ -182,15 +182,16 @@ static inline size_t prefill_part_bytes(int batch, int nsplit, int l) {
 // leave no share of the last tile empty are looked at.
 // Measured with every split over 2 to 4096 tokens, 0 to 60000 cached, 1 and 2 rows of Q4K, Q8_0
 // and F16 (696 shapes): the split taken is 0.4% slower than the best one in the mean, over 10%
-// in 4 shapes. Whole rounds of mean workgroups and merges twice as dear had 1.3% and 32 (Q8_0
+// in 3 shapes. Whole rounds of mean workgroups and merges twice as dear had 1.3% and 32 (Q8_0
 // 700 tokens after 500 64.1 us at 3 splits, 72.3 at the 2 taken then). A few tokens over a
 // long cache take as many splits as give every CU a workgroup: 5 tokens over 20016 keys 98.8 us
 // at 16 splits, 24.5 at 126. The partials take kPfMaxPartBytes at most: beyond lie chunks of
 // many rows that fill the GPU without a split.
 static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk) {
-  constexpr double kPfFixed = 2.5;  // q, the first block's latency, the epilogue
-  // bytes of partials in a block's time; twice the time for those past kMergeNear
-  constexpr double kMergeFixed = 2.5, kMergeBytes = 8e6, kMergeNear = 64e6;
+  constexpr double kPfFixed = 3.5;  // q, the first block's latency, the epilogue
+  // the merge's launch, and bytes of partials in a block's time: fewer where one round of
+  // workgroups writes them at its end, half past kMergeNear
+  constexpr double kMergeFixed = 0.9, kMergeBytes1 = 5e6, kMergeBytes = 8e6, kMergeNear = 64e6;
   // blocks of the first and the last tile (the causal limit cuts the first ones')
   int nb0 = nblk, nb1 = nblk;
   if (a.causal) {
@@ -214,7 +215,9 @@ static inline int prefill_splits(const AttnArgs &a, int ntiles, int nblk) {
       const double sum = (full - 1) * 0.5 * (longest + length(full - 1)) + 2 * length(full);
       t = sum > t ? sum : t;
     }
-    if (ns > 1) t += kMergeFixed + (bytes + (bytes > kMergeNear ? bytes - kMergeNear : 0.0)) / kMergeBytes;
+    if (ns > 1)
+      t += kMergeFixed + bytes / (wgs <= kPfTargetWGs ? kMergeBytes1 : kMergeBytes) +
+           (bytes > kMergeNear ? (bytes - kMergeNear) / kMergeBytes : 0.0);
     if (t < best_t) {
       best_t = t;
       best = ns;
