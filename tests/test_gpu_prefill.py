@@ -175,7 +175,7 @@ def test_prefill_full_chunk(pk, orc, quant):
 @pytest.mark.parametrize("quant", QUANTS)
 @pytest.mark.parametrize("L", [12, 33, 64, 100])
 def test_prefill_wide_merges(pk, orc, L, quant):
-    """Up to 126, 42, 32 and 18 key splits: every form of the wide merge."""
+    """84, 42, 32 and 17 key splits: every form of the wide merge."""
     say(f"prefill wide merge quant={quant} L={L}")
     run_prefill(pk, orc, 8000, L, seed=900 + L, quant=quant)
 
